@@ -165,9 +165,9 @@ int lstk_moe_route(lstk_pool *pool, int layer, const float *d_hnorm, int n_token
  * the weight type (Q8_0 for Q8_0, Q8_K for Q4_K), and so is the SwiGLU output before down.
  * d_slots holds slot numbers from lstk_pool_acquire (streaming) or expert ids (resident).
  * d_out may alias d_resid.
- * With Q4_K gate, up and down and at least 64 tokens (LSTK_GROUPED_MIN_TOKENS in the environment
- * overrides the threshold) the call takes the grouped path: a stable permutation of the pairs by
- * expert, then expert products on the matrix cores over 64-pair chunks. */
+ * From 32 tokens on (49 with Q4_K gate, up and down; LSTK_GROUPED_MIN_TOKENS in the environment overrides the
+ * threshold) the call takes the grouped path: a stable permutation of the pairs by expert, then expert products
+ * on the matrix cores over chunks of 16 or 32 pairs. */
 int lstk_moe_ffn(lstk_pool *pool, int layer, const float *d_hnorm, const int32_t *d_slots, const float *d_weights,
                  const float *d_resid, float *d_out, int n_tokens, lstk_stream_t stream);
 

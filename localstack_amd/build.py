@@ -14,7 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "liblstk_moe.so")
-SOURCES = ["kernels.hip", "grouped.hip", "fused.hip", "forward.hip", "pool.cpp", "repack.cpp", "model.cpp", "gguf.cpp", "tier.hip"]
+SOURCES = ["kernels.hip", "grouped.hip", "grouped_rows.hip", "fused.hip", "forward.hip", "pool.cpp", "repack.cpp", "model.cpp", "gguf.cpp", "tier.hip"]
 ARCH = os.environ.get("LSTK_OFFLOAD_ARCH", "gfx950")
 
 
@@ -27,7 +27,7 @@ def hipcc():
 
 # Per-source extra flags. The grouped MFMA kernels keep their accumulators in VGPRs (the VALU
 # epilogue then reads them without v_accvgpr_read moves).
-EXTRA = {"grouped.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+EXTRA = {s: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for s in ("grouped.hip", "grouped_rows.hip")}
 COMMON = ["-O3", "-std=c++20", "-fPIC",
           # packed-FP32 instructions off for all device code
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

@@ -149,6 +149,7 @@ __global__ __launch_bounds__(kPermThreads) void permute_kernel(PermuteParams P) 
     if (tid < nb) {
         P.counts[tid] = c;
         P.offsets[tid] = off;
+        if (P.limit > 0 && c > P.limit) atomicOr(P.err, 2);
         if (P.items) {
             // expert-major: a bin's chunks are consecutive items (XCD-aware mapping keeps them on one XCD)
             const int fb = b1 + v1 - nch;
@@ -559,20 +560,21 @@ __global__ __launch_bounds__(kGThreads, LSTK_GROUPED_MIN_WAVES) void down_groupe
     }
 }
 
+template <int QT>
 __global__ __launch_bounds__(128) void act_quant_kernel(const float *act, int f, int8_t *qs, float *d, int32_t *bs,
                                                         uint32_t *bh) {
     const size_t p = blockIdx.x;
-    quantize_row<kTypeQ4_K>(act + p * f, f, qs + p * f, d + p * (f / 32), bs + p * (f / 32), bh + p * (f / 32));
+    quantize_row<QT>(act + p * f, f, qs + p * f, d + p * (f / 32), bs + p * (f / 32), bh + p * (f / 32));
 }
 
 }  // namespace
 
 bool grouped_supported(int tu, int tg, int td, int h, int f, int n_bins) {
-    return tu == kTypeQ4_K && tg == kTypeQ4_K && td == kTypeQ4_K && h % 256 == 0 && f % 256 == 0 && f % 64 == 0 &&
-           n_bins >= 1 && n_bins <= kGroupedMaxBins;
+    return tu == tg && supported_weight_type(tg) && supported_weight_type(td) && h % 256 == 0 && f % 256 == 0 && n_bins >= 1 &&
+           n_bins <= kGroupedMaxBins;
 }
 
-int grouped_max_items(int np, int n_bins) { return (np + kGroupedChunk - 1) / kGroupedChunk + std::min(n_bins, np); }
+int grouped_max_items(int np, int n_bins, int chunk) { return (np + chunk - 1) / chunk + std::min(n_bins, np); }
 
 hipError_t launch_permute(const PermuteParams &P, hipStream_t st, const LaunchTiming *tm) {
     if (P.np <= 0) return hipSuccess;
@@ -609,10 +611,11 @@ hipError_t launch_down_grouped(const GroupedParams &P, int max_items, hipStream_
     return launch(down_grouped_kernel, dim3(kXcds * per * (P.rows / 128)), dim3(kGThreads), kGLdsBytes, st, tm, P);
 }
 
-hipError_t launch_act_quant(const float *act, int f, int np, const ActBuf &aq, hipStream_t st, const LaunchTiming *tm) {
+hipError_t launch_act_quant(const float *act, int f, int np, int qtype, const ActBuf &aq, hipStream_t st, const LaunchTiming *tm) {
     if (np <= 0) return hipSuccess;
     if (!aq.bh) return hipErrorInvalidValue;
-    return launch(act_quant_kernel, dim3(np), dim3(128), 0, st, tm, act, f, aq.qs, aq.d, aq.bs, aq.bh);
+    return qtype == kTypeQ8_0 ? launch(act_quant_kernel<kTypeQ8_0>, dim3(np), dim3(128), 0, st, tm, act, f, aq.qs, aq.d, aq.bs, aq.bh)
+                              : launch(act_quant_kernel<kTypeQ4_K>, dim3(np), dim3(128), 0, st, tm, act, f, aq.qs, aq.d, aq.bs, aq.bh);
 }
 
 }  // namespace lstk

@@ -126,6 +126,7 @@ struct PermuteParams {
     int4 *items;      // [max_items] {bin, first position, pairs, 0}: each bin's chunks in order, bins ascending; may be null
     int32_t *n_items; // may be null
     int32_t *err;
+    int limit;        // > 0: a bin with more pairs sets bit 2 of *err (as the GEMV path's kernels do past T)
 };
 
 // One grouped expert product over the work list: Q4_K weight rows x Q8_K activation rows on MFMA.
@@ -145,6 +146,8 @@ struct GroupedParams {
     int row_div;             // activation row = pair / row_div
     const float *weights;    // down: router weight of each pair
     float *out;
+    int type;                // ggml type of the weights
+    int chunk;               // pairs per work item
 };
 
 // The whole MoE block of one token in one launch (fused.hip). Work-groups [0, nB) each compute one
@@ -245,11 +248,15 @@ constexpr int kGroupedMaxBins = 1024;    // bins the permutation kernel handles
 // n_bins <= kGroupedMaxBins.
 bool grouped_supported(int tu, int tg, int td, int h, int f, int n_bins);
 // Upper bound on the work items of np pairs over n_bins bins.
-int grouped_max_items(int np, int n_bins);
+int grouped_max_items(int np, int n_bins, int chunk);
 hipError_t launch_permute(const PermuteParams &p, hipStream_t s, const LaunchTiming *t);
 hipError_t launch_gate_up_grouped(const GroupedParams &p, int max_items, hipStream_t s, const LaunchTiming *t);
-hipError_t launch_act_quant(const float *act, int f, int np, const ActBuf &aq, hipStream_t s, const LaunchTiming *t);
+// qtype 8: Q8_0 rows, otherwise Q8_K rows.
+hipError_t launch_act_quant(const float *act, int f, int np, int qtype, const ActBuf &aq, hipStream_t s, const LaunchTiming *t);
 hipError_t launch_down_grouped(const GroupedParams &p, int max_items, hipStream_t s, const LaunchTiming *t);
+// The same products for every pool format with the weights streamed through registers, grouped_rows.hip.
+hipError_t launch_gate_up_rows(const GroupedParams &p, int max_items, hipStream_t s, const LaunchTiming *t);
+hipError_t launch_down_rows(const GroupedParams &p, int max_items, hipStream_t s, const LaunchTiming *t);
 
 // fused single-token path, fused.hip
 FusedLayout fused_layout(int h, int f, int E, int k);

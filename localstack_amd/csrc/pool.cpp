@@ -225,7 +225,7 @@ int alloc_scratch(lstk_pool *P) {
     const size_t o_act = take(T * k * f * 4), o_Y = take(T * k * h * 4);
     const size_t o_err = take(64);
     const size_t np = T * k;
-    const size_t max_items = (size_t) lstk::grouped_max_items((int) np, (int) nb);
+    const size_t max_items = (size_t) lstk::grouped_max_items((int) np, (int) nb, 16);
     const size_t o_counts = take(nb * 4), o_offsets = take((nb + 1) * 4), o_perm = take(np * 4), o_nitems = take(64);
     const size_t o_items = take(max_items * 16);
     const size_t o_aqs = take(np * f), o_ad = take(np * (f / 32) * 4), o_abs = take(np * (f / 32) * 4);
@@ -833,26 +833,49 @@ int check_call(lstk_pool *P, int layer, int T) {
     return LSTK_OK;
 }
 
-// The grouped MFMA path serves calls with many tokens per expert (prefill): Q4_K gate, up and down,
-// at least grouped_min_tokens tokens (LSTK_GROUPED_MIN_TOKENS overrides the default of 64).
+// The matrix-core path of many-token calls. A call takes it from T tokens on (LSTK_GROUPED_MIN_TOKENS overrides):
+// 32 with Q8_0 or KQ8 experts, 49 with Q4_K gate, up and down. Measured on one 30B-shaped layer, GEMV path against this
+// one, us a layer with even / Zipf(1.1) routing: Q8_0 24 tokens 101 / 112, 32 tokens 118 / 126 and 114 / 59, 48 tokens
+// 147 / 140; Q2_K + Q3_K 17 tokens 107 / 112, 32 tokens 144 / 136; Q4_K + Q6_K 32 tokens 110 / 100; Q4_K 50 tokens
+// 127 / 94 and 152 / 57 (up to 48 Q4_K tokens stay where lstk_moe_block_noalloc is bit-identical to lstk_moe_block).
+constexpr int kGroupedMinTokens = 32, kGroupedMinTokensQ4K = 49;
 bool use_grouped(lstk_pool *P, const Shard &s, int T) {
     if (P->grouped_min_tokens == 0) {
         const char *env = std::getenv("LSTK_GROUPED_MIN_TOKENS");
-        P->grouped_min_tokens = env ? std::max(1, std::atoi(env)) : 64;
+        P->grouped_min_tokens = env ? std::max(1, std::atoi(env)) : -1;
     }
-    return T >= P->grouped_min_tokens &&
-           lstk::grouped_supported(s.tu, s.tg, s.td, P->dims.n_embd, P->dims.n_ff_exp, (int) s.n_slots);
+    const bool q4k = s.tg == lstk::kTypeQ4_K && s.td == lstk::kTypeQ4_K;
+    const int from = P->grouped_min_tokens > 0 ? P->grouped_min_tokens : q4k ? kGroupedMinTokensQ4K : kGroupedMinTokens;
+    return T >= from && lstk::grouped_supported(s.tu, s.tg, s.td, P->dims.n_embd, P->dims.n_ff_exp, (int) s.n_slots);
 }
 
-// permute -> gate_up (MFMA, SwiGLU) -> Q8_K of the SwiGLU rows -> down (MFMA, router weight) ->
+// Which kernels run a many-token call's expert products, and the pairs per work item.
+// rows (grouped_rows.hip): every format; for Q4_K alone up to 14 pairs per expert (one 30B-shaped layer, LDS-staged
+//   kernels of grouped.hip against rows, us: 64 tokens 106 / 98, 128 115 / 103, 203 122 / 113, 256 123 / 126, 512 166 / 180;
+//   the staged kernels build their weight planes once per 32 pairs and win when the pairs fill them).
+// chunk: 16 pairs (one matrix-core tile, 36 KB of LDS at h 2048) or, for Q8_0 past 12 pairs per expert, 32 (us: 200
+//   tokens 165 / 165, 256 181 / 174, 400 214 / 199, 300 Zipf-routed 153 / 137). KQ8 stays at 16: its second tile takes
+//   the kernel past 200 VGPRs (203 tokens 135 / 200).
+struct GroupedPlan {
+    bool rows;
+    int chunk;
+};
+GroupedPlan grouped_plan(const Shard &s, int np, int n_expert) {
+    if (s.tg == lstk::kTypeQ4_K && s.td == lstk::kTypeQ4_K && np > 14 * n_expert) return {false, lstk::kGroupedChunk};
+    const bool q8 = s.tg == lstk::kTypeQ8_0 && s.td == lstk::kTypeQ8_0;
+    return {true, q8 && np > 12 * n_expert ? 32 : 16};
+}
+
+// permute -> gate_up (MFMA, SwiGLU) -> Q8_0 / Q8_K of the SwiGLU rows -> down (MFMA, router weight) ->
 // combine + residual. bins: expert ids (resident) or slots (streaming), [T][k].
 int run_grouped(lstk_pool *P, const Shard &s, const int32_t *bins, const float *d_weights, const float *d_resid,
                 float *d_out, int T, hipStream_t st) {
     const lstk_moe_dims &d = P->dims;
     const int k = d.n_expert_used, np = T * k, h = d.n_embd, f = d.n_ff_exp;
-    const int max_items = lstk::grouped_max_items(np, (int) s.n_slots);
-    lstk::PermuteParams pp{bins, np, (int) s.n_slots, lstk::kGroupedChunk, P->counts, P->offsets, P->perm,
-                           P->items, P->n_items, P->err};
+    const auto [rows, chunk] = grouped_plan(s, np, d.n_expert);
+    const int max_items = lstk::grouped_max_items(np, (int) s.n_slots, chunk);
+    lstk::PermuteParams pp{bins, np, (int) s.n_slots, chunk, P->counts, P->offsets, P->perm,
+                           P->items, P->n_items, P->err, s.tg == lstk::kTypeQ4_K && s.td == lstk::kTypeQ4_K ? 0 : T};
     hipError_t e = timed(P, 0, [&](const lstk::LaunchTiming *tm) { return lstk::launch_permute(pp, st, tm); });
     if (e != hipSuccess) return hip_fail(e, "permute launch");
     lstk::GroupedParams gu{};
@@ -871,9 +894,13 @@ int run_grouped(lstk_pool *P, const Shard &s, const int32_t *bins, const float *
     gu.xbh = P->xq.bh;
     gu.row_div = k;
     gu.out = P->act;
-    e = timed(P, 1, [&](const lstk::LaunchTiming *tm) { return lstk::launch_gate_up_grouped(gu, max_items, st, tm); });
+    gu.type = s.tg;
+    gu.chunk = chunk;
+    e = timed(P, 1, [&, rows = rows](const lstk::LaunchTiming *tm) {
+        return rows ? lstk::launch_gate_up_rows(gu, max_items, st, tm) : lstk::launch_gate_up_grouped(gu, max_items, st, tm);
+    });
     if (e != hipSuccess) return hip_fail(e, "gate_up launch");
-    e = timed(P, 2, [&](const lstk::LaunchTiming *tm) { return lstk::launch_act_quant(P->act, f, np, P->aq, st, tm); });
+    e = timed(P, 2, [&](const lstk::LaunchTiming *tm) { return lstk::launch_act_quant(P->act, f, np, s.td, P->aq, st, tm); });
     if (e != hipSuccess) return hip_fail(e, "act quant launch");
     lstk::GroupedParams dn = gu;
     dn.w0 = s.d_down;
@@ -888,7 +915,10 @@ int run_grouped(lstk_pool *P, const Shard &s, const int32_t *bins, const float *
     dn.row_div = 1;
     dn.weights = d_weights;
     dn.out = P->Y;
-    e = timed(P, 2, [&](const lstk::LaunchTiming *tm) { return lstk::launch_down_grouped(dn, max_items, st, tm); });
+    dn.type = s.td;
+    e = timed(P, 2, [&, rows = rows](const lstk::LaunchTiming *tm) {
+        return rows ? lstk::launch_down_rows(dn, max_items, st, tm) : lstk::launch_down_grouped(dn, max_items, st, tm);
+    });
     if (e != hipSuccess) return hip_fail(e, "down launch");
     if (P->defer_combine) return LSTK_OK;
     lstk::CombineParams cp{P->Y, d_resid, d_out, T, k, h};

@@ -1,0 +1,58 @@
+"""GPU parity of the many-token expert kernels that stream their weights through registers (grouped_rows.hip) against
+the oracle: every expert format, pair counts per expert at the edges of a 16- and a 32-pair work item (0, 1, 15, 16,
+17, 31, 32, 33), one and many super-blocks per row, and the two activation types in one layer.
+
+Bar: the one of the other expert kernels (test_gpu_grouped.py): 2e-3 of the largest |out - resid|, for the f32 order
+over super-blocks, expf, and a SwiGLU value that rounds the other way into its 8 bits. Such a value moves an output by
+one 8-bit step of one of f products, so against outputs that grow as sqrt(f) its share grows as 1 / sqrt(f): the bar,
+set at f >= 512, is 2e-3 sqrt(512 / f) below that (2.8e-3 at f 256; measured up to 2.02e-3 there).
+"""
+import numpy as np
+import pytest
+
+from localstack_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+FFN_TOL = 2e-3
+# expert: pairs of 64 tokens, two columns of distinct experts per token
+COUNTS = ((1, 15, 16, 32), (17, 33, 14, 0))
+
+
+def _ids(rng, T, reps):
+    """ids [T, 2]: column c holds expert 4 c + i COUNTS[c][i] * reps times, shuffled."""
+    cols = [np.repeat(np.arange(4 * c, 4 * c + 4), np.array(n) * reps) for c, n in enumerate(COUNTS)]
+    for c in cols:
+        rng.shuffle(c)
+    return np.stack(cols, 1)[:T].astype(np.int32)
+
+
+@pytest.mark.parametrize("types,h,f,T", [
+    ((8, 8, 8), 256, 256, 64), ((8, 8, 8), 256, 512, 320), ((8, 8, 8), 4096, 512, 64), ((8, 8, 8), 4096, 256, 64 * 3),
+    ((12, 12, 12), 256, 256, 64), ((12, 12, 12), 4096, 256, 64), ((10, 10, 11), 256, 512, 64), ((11, 11, 10), 512, 256, 63),
+    ((13, 13, 14), 512, 256, 64), ((14, 14, 13), 256, 256, 33), ((12, 12, 14), 2048, 768, 64), ((12, 12, 8), 512, 256, 64),
+    ((8, 8, 14), 256, 256, 320), ((10, 10, 11), 4096, 256, 64),
+], ids=lambda v: "-".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_rows_ffn_matches_oracle(orc, lstk, dev, types, h, f, T):
+    import torch
+    E, k = 16, 2  # experts 8 .. 15 stay idle; 64 tokens take 16-pair items, more take 32 with Q8_0
+    rng = np.random.default_rng(100 * types[0] + types[2] + h + f + T)
+    up, gate, down = (synth.experts(rng, types[0], E, f, h, centered=True), synth.experts(rng, types[1], E, f, h, centered=True),
+                      synth.experts(rng, types[2], E, h, f, centered=True))
+    x, resid = synth.activations(rng, T, h), synth.activations(rng, T, h)
+    ids = _ids(rng, T, -(-T // 64))
+    w = rng.uniform(0.1, 0.9, (T, k)).astype(np.float32)
+    store = lstk.ExpertStore(1, h, f, E, k, T, [(types, up, gate, down)])
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    outs = []
+    for _ in range(2):
+        out = torch.full((T, h), np.nan, dtype=torch.float32, device=dev)
+        store.ffn(0, d(x), d(ids), d(w), d(resid), out)
+        store.check()
+        outs.append(out.cpu().numpy())
+    store.close()
+    assert np.array_equal(outs[0], outs[1]), "repeated calls differ"
+    ref = orc.moe_ffn(x, ids, w, resid, up.reshape(E, -1), gate.reshape(E, -1), down.reshape(E, -1), types, f)
+    err = np.abs(outs[0] - ref).max() / np.abs(ref - resid).max()
+    print(f"[rows {types} h={h} f={f} T={T}] rel max err {err:.3e}", flush=True)
+    assert err <= FFN_TOL * max(1.0, (512 / f) ** 0.5)
