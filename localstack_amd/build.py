@@ -27,7 +27,7 @@ def hipcc():
 
 # Per-source extra flags. The grouped MFMA kernels keep their accumulators in VGPRs (the VALU
 # epilogue then reads them without v_accvgpr_read moves).
-EXTRA = {s: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for s in ("grouped.hip", "grouped_rows.hip")}
+EXTRA = {s: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for s in ("grouped.hip", "grouped_rows.hip", "forward.hip")}
 COMMON = ["-O3", "-std=c++20", "-fPIC",
           # packed-FP32 instructions off for all device code
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

@@ -1045,7 +1045,7 @@ __global__ __launch_bounds__(NW *kWave) void attn1_kernel(AttnParams P) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// Attention of 64-row blocks (steps of many tokens): wavefront w owns query rows row0 + 16 w .. + 15
+// Attention of 64-row blocks (steps of 8 to 63 tokens at 8 query heads per KV head): wavefront w owns query rows row0 + 16 w .. + 15
 // over the whole chunk and runs them from registers to registers as attn1_kernel does (S^T = K Q^T puts
 // a row's scores in that row's lanes, the online softmax stays there, O^T += V^T P^T with P as fp16
 // hi + lo). The K and V fragments of each 64-cell block (and its cell-table entries) are loaded once
@@ -1053,13 +1053,12 @@ __global__ __launch_bounds__(NW *kWave) void attn1_kernel(AttnParams P) {
 // wavefronts read them; the next live block's loads are in flight while a block is multiplied. Two
 // barriers per 64-cell block; no score or probability goes through LDS.
 // ------------------------------------------------------------------------------------------------
-template <int HD, bool SKIP>
+template <int HD>
 __global__ __launch_bounds__(kAtBlock) void attn_rows_kernel(AttnParams P) {
     constexpr int NK = HD / 16;
     __shared__ __align__(16) half4v s_k[4][NK][kWave];
     __shared__ __align__(16) half4v s_v[4][NK][kWave];
     __shared__ __align__(16) int s_cs[kFaCells], s_cp[kFaCells];
-    __shared__ uint8_t s_live[SKIP ? kAttnMaxPasses : 1];
     const int tid = threadIdx.x, w = tid / kWave, l = tid & (kWave - 1), lr = l & 15, lq = l >> 4;
     const int grp = P.n_head / P.n_kv;
     const int g = blockIdx.x % P.n_kv, rest = blockIdx.x / P.n_kv;
@@ -1086,22 +1085,6 @@ __global__ __launch_bounds__(kAtBlock) void attn_rows_kernel(AttnParams P) {
         const int ct = min(b0 + 16 * w + (l & 15), P.kv_size - 1);
         ctr = l < 16 ? P.cell_seq[ct] : P.cell_pos[ct];
     };
-    // A step of many tokens skips the chunk's passes that hold no cell of the sequence (attn_kernel's map)
-    const bool skip = SKIP && n_pass <= kAttnMaxPasses;
-    if (skip) {
-        for (int p0 = 0; p0 < n_pass; p0 += 8 * (kAtBlock / kWave)) {
-            int cs[8];
-#pragma unroll
-            for (int u = 0; u < 8; u++) cs[u] = P.cell_seq[min(begin + (p0 + u * (kAtBlock / kWave) + w) * kFaCells + l, P.kv_size - 1)];
-#pragma unroll
-            for (int u = 0; u < 8; u++) {
-                const int pass = p0 + u * (kAtBlock / kWave) + w;
-                const bool mine = cs[u] == P.seq && begin + pass * kFaCells + l < end;
-                const bool any = __ballot(mine) != 0ull;
-                if (l == 0 && pass < n_pass) s_live[pass] = any ? 1 : 0;
-            }
-        }
-    }
     half4v qb[NK];
     const uint16_t *q = P.q + ((size_t) t * P.n_head + h) * HD;
 #pragma unroll
@@ -1109,13 +1092,7 @@ __global__ __launch_bounds__(kAtBlock) void attn_rows_kernel(AttnParams P) {
         const half4v v = ld_half4(q + ks * 16 + 4 * lq);
         qb[ks] = on ? v : half4v{0, 0, 0, 0};
     }
-    __syncthreads(); // the skip map
-    auto next_live = [&](int p) {
-        if (skip)
-            while (p < n_pass && !s_live[p]) p++;
-        return p;
-    };
-    int p = next_live(0);
+    int p = 0;
     load_block(begin + min(p, n_pass - 1) * kFaCells);
     float m_run = -INFINITY, l_run = 0.0f;
     f32x4v o[NK];
@@ -1131,7 +1108,7 @@ __global__ __launch_bounds__(kAtBlock) void attn_rows_kernel(AttnParams P) {
         if (l < 16) s_cs[16 * w + l] = ctr;
         else if (l < 32) s_cp[16 * w + l - 16] = ctr;
         __syncthreads();
-        const int pn = next_live(p + 1);
+        const int pn = p + 1;
         load_block(begin + min(pn, n_pass - 1) * kFaCells); // unconditional: the last block again past the end
         // the block's four 16-cell groups together: S^T of each (four independent product chains), one
         // softmax step over the 64 cells, then O^T += V^T P^T over the groups (eight chains, one per dim tile)
@@ -1215,14 +1192,291 @@ __global__ __launch_bounds__(kAtBlock) void attn_rows_kernel(AttnParams P) {
     }
 }
 
+// ------------------------------------------------------------------------------------------------
+// Prompt attention (steps of many tokens in 64-row blocks). The work-group's eight wavefronts split the cells, not the
+// rows: a wavefront takes every eighth 16-cell unit of the chunk for all 64 rows, with its K and V fragments loaded
+// straight from the cache into registers (the cache layout is the operand layout) and the rows' Q fragments read from
+// LDS. Each keeps a running maximum, sum and output of all 64 rows for its own cells, so nothing is exchanged and no
+// barrier is met until the end, where the eight partial rows are summed through LDS. A prompt's launch is about one
+// work-group per CU: with the rows split instead (attn_rows_kernel) a SIMD held one wavefront, and every LDS read,
+// product chain and exponential of a block waited in line; here it holds two with 4 and 32 independent product chains.
+// A unit's next K is requested when its scores are done, its next V when its products are.
+//
+// A 32-cell block is live for the work-group when some cell of it belongs to the sequence at a position its last row
+// sees: other sequences' blocks and those above the causal diagonal cost nothing. The live blocks are taken in the
+// order of their positions (a block holds consecutive positions of one sequence from its first cell), so a chunk's sums
+// do not depend on the order its blocks lie in. Where a unit is seen whole (every
+// cell the sequence's, none past the row block's first row) its scores skip the visibility tests.
+//
+// The softmax runs in base 2 against a running maximum raised to the next integer: p = 2^(s c - m) with c = scale log2 e
+// is one fma and one hardware exponential per score, and a row's rescale between maxima is an exact power of two. The
+// products are 32 deep (16 x 16 x 32): two 16-dim steps of a score in one, and p's hi and lo parts against the same V in
+// one; their sums are as close to 64 bits as the 16-deep form's (1e-8 .. 3e-8 of sum |a b| on random and on softmax-like
+// operands, both).
+//
+// Bound: VALU and matrix-core issue, about 0.8k cycles each per unit. 512 tokens after 3584 at the 30B shape: 215 -> 78 us
+// a launch (256 work-groups on MI355X), after 512 55 -> 31 us, no context 35 -> 21 us.
+// ------------------------------------------------------------------------------------------------
+
+// The two values a lane and its partner 16 (or 32) lanes away hold, in the same order in both lanes.
+__device__ __forceinline__ float2 both16(float v) {
+    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return make_float2(__uint_as_float(p[0]), __uint_as_float(p[1]));
+}
+__device__ __forceinline__ float2 both32(float v) {
+    const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return make_float2(__uint_as_float(p[0]), __uint_as_float(p[1]));
+}
+
+typedef _Float16 half8v __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ half8v join(half4v a, half4v b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
+__device__ __forceinline__ f32x4v mfma32(half8v a, half8v b, f32x4v c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+
+constexpr int kAsMapBlocks = 2 * kAttnMaxPasses; // 32-cell blocks a chunk's map covers
+constexpr int kAsWaves = 8, kAsCells = 16; // wavefronts of a work-group, cells per unit
+template <int HD>
+struct AttnSplitLds {
+    static constexpr int NK = HD / 16;
+    union {
+        uint16_t at[kAsMapBlocks];            // the live block of each position / 32 (of each block index past 131072 cells)
+        f32x4v o[kAsWaves][4][NK / 2][kWave]; // at the end: half of the dims of the wavefronts' outputs at a time
+    };
+    half8v q[4][NK / 2][kWave]; // the rows' Q fragments, two 16-dim steps side by side
+    float m[kAsWaves][64], l[kAsWaves][64];
+    uint16_t list[kAsMapBlocks]; // the live blocks in order
+    int n_live;
+};
+
+template <int HD>
+__global__ __launch_bounds__(kAsWaves *kWave) void attn_split_kernel(AttnParams P) {
+    constexpr int NK = HD / 16;
+    extern __shared__ __align__(16) unsigned char smem_split[];
+    auto &S = *reinterpret_cast<AttnSplitLds<HD> *>(smem_split);
+    const int tid = threadIdx.x, l = tid & (kWave - 1), lr = l & 15, lq = l >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int grp = P.n_head / P.n_kv;
+    const int g = blockIdx.x % P.n_kv, rest = blockIdx.x / P.n_kv;
+    const int c = rest % P.n_chunk, rb = rest / P.n_chunk;
+    const int rows = P.T * grp;
+    const int begin = P.cell_begin + c * P.chunk, end = min(begin + P.chunk, P.n_cells);
+    const int n_pass = (end - begin + kFaCells - 1) / kFaCells;
+    // positions rise over a step's tokens
+    const int pos_first = P.pos[rb * 64 / grp], pos_last = P.pos[min(rb * 64 + 63, rows - 1) / grp];
+    // the lane's rows: row lr of each 16-row tile (B operand of S^T); rows past the end read the last row, see no cell
+    // and store nothing
+    int pos[4];
+#pragma unroll
+    for (int rt = 0; rt < 4; rt++) {
+        const int r = rb * 64 + 16 * rt + lr, t = min(r, rows - 1) / grp;
+        pos[rt] = r < rows ? P.pos[t] : -1;
+    }
+    for (int i = wave; i < 4 * (NK / 2); i += kAsWaves) {
+        const int rt = i / (NK / 2), k2 = i % (NK / 2), r = rb * 64 + 16 * rt + lr, rc = min(r, rows - 1);
+        const uint16_t *q = P.q + ((size_t) (rc / grp) * P.n_head + g * grp + rc % grp) * HD + k2 * 32 + 4 * lq;
+        const half8v v = join(ld_half4(q), ld_half4(q + 16));
+        S.q[rt][k2][l] = r < rows ? v : half8v{0, 0, 0, 0, 0, 0, 0, 0};
+    }
+    const bool skip = n_pass <= kAttnMaxPasses; // (beyond the map every cell is taken, in order)
+    if (skip) {
+        const bool by_pos = P.kv_size <= 32 * kAsMapBlocks;
+        const int n_at = by_pos ? min(pos_last / 32 + 1, kAsMapBlocks) : 2 * n_pass;
+        for (int i = tid; i < n_at; i += kAsWaves * kWave) S.at[i] = 0xffffu;
+        __syncthreads();
+        for (int p0 = 0; p0 < n_pass; p0 += 4 * kAsWaves) {
+            int cs[4], cp[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int cell = min(begin + (p0 + u * kAsWaves + wave) * kFaCells + l, P.kv_size - 1);
+                cs[u] = P.cell_seq[cell];
+                cp[u] = P.cell_pos[cell];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int pass = p0 + u * kAsWaves + wave;
+                const unsigned long long mk =
+                    __ballot(pass < n_pass && cs[u] == P.seq && cp[u] <= pos_last && begin + pass * kFaCells + l < end);
+                const int blk = 2 * pass + (l >> 5), key = by_pos ? cp[u] / 32 : blk;
+                // (lanes 0 and 32: their cells are the blocks' first, with the lowest positions)
+                if ((l & 31) == 0 && (unsigned) (mk >> (l & 32)) != 0u && key >= 0 && key < n_at) S.at[key] = (uint16_t) blk;
+            }
+        }
+        __syncthreads();
+        if (wave == 0) {
+            int n = 0;
+            for (int i0 = 0; i0 < n_at; i0 += kWave) {
+                const unsigned blk = i0 + l < n_at ? S.at[i0 + l] : 0xffffu;
+                const unsigned long long mk = __ballot(blk != 0xffffu);
+                if (blk != 0xffffu) S.list[n + __popcll(mk & ((1ull << l) - 1ull))] = (uint16_t) blk;
+                n += __popcll(mk);
+            }
+            if (l == 0) S.n_live = n;
+        }
+    }
+    __syncthreads();
+    const int n_unit = skip ? 2 * S.n_live : n_pass * (kFaCells / kAsCells);
+    // first cell of unit u; past the end the last unit's (loaded again and not multiplied)
+    auto unit_cell = [&](int u) {
+        u = min(u, n_unit - 1);
+        return begin + (skip ? (int) __builtin_amdgcn_readfirstlane((int) S.list[u / 2]) * 32 + (u % 2) * kAsCells : u * kAsCells);
+    };
+    half4v kr[NK], vr[NK]; // K of cell lr of the unit, V of cells 4 lq .. + 3
+    int seen;              // lanes 0-15: the position of cell l of the unit, INT_MAX if it is not the sequence's
+    // a scalar base per fragment and one 32-bit offset per lane (a head's cache stays below 4 GB)
+    const uint8_t *kp = reinterpret_cast<const uint8_t *>(P.kc + (size_t) g * HD * P.kv_size);
+    const uint8_t *vp = reinterpret_cast<const uint8_t *>(P.vc + (size_t) g * HD * P.kv_size);
+    auto load_k = [&](int b0) {
+        const int ct = b0 + lr, cc = min(ct, P.kv_size - 1);
+        const int cs = P.cell_seq[cc], cp = P.cell_pos[cc];
+        const unsigned ok = (unsigned) (lq * P.kv_size + cc) * 8;
+#pragma unroll
+        for (int ks = 0; ks < NK; ks++)
+            kr[ks] = __builtin_bit_cast(half4v, *reinterpret_cast<const uint2 *>(kp + (size_t) ks * 32 * P.kv_size + ok));
+        seen = cs == P.seq && ct < end ? cp : INT_MAX;
+    };
+    auto load_v = [&](int b0) {
+        const unsigned ov = (unsigned) (min(b0 + 4 * lq, P.kv_size - 4) / 4 * HD + lr) * 8;
+#pragma unroll
+        for (int dt = 0; dt < NK; dt++) vr[dt] = __builtin_bit_cast(half4v, *reinterpret_cast<const uint2 *>(vp + 128 * dt + ov));
+    };
+    const float c2 = (float) ((double) P.scale * 1.44269504088896340736);
+    float m[4], lsum[4]; // m: an integer, or -inf before a row sees a cell
+    f32x4v o[4][NK];
+#pragma unroll
+    for (int rt = 0; rt < 4; rt++) {
+        m[rt] = -INFINITY;
+        lsum[rt] = 0.0f;
+#pragma unroll
+        for (int dt = 0; dt < NK; dt++) o[rt][dt] = f32x4v{0, 0, 0, 0};
+    }
+    if (wave < n_unit) {
+        const int b0 = unit_cell(wave);
+        load_k(b0);
+        load_v(b0);
+    }
+    for (int u = wave; u < n_unit; u += kAsWaves) {
+        asm volatile("" ::: "memory"); // the Q fragments are read again per unit (held across units, 64 registers would spill)
+        f32x4v sc[4];
+#pragma unroll
+        for (int rt = 0; rt < 4; rt++) sc[rt] = f32x4v{0, 0, 0, 0};
+#pragma unroll
+        for (int k2 = 0; k2 < NK / 2; k2++) {
+            const half8v kf = join(kr[2 * k2], kr[2 * k2 + 1]);
+#pragma unroll
+            for (int rt = 0; rt < 4; rt++) sc[rt] = mfma32(kf, S.q[rt][k2][l], sc[rt]);
+        }
+        const int see = seen, bn = unit_cell(u + kAsWaves);
+        load_k(bn);
+        if (__ballot(see > pos_first) != 0ull) {
+            // some cell is hidden from some row: lane (lr, lq) holds cells 4 lq + v
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int cp = __shfl(see, 4 * lq + v, kWave);
+#pragma unroll
+                for (int rt = 0; rt < 4; rt++) sc[rt][v] = cp <= pos[rt] ? sc[rt][v] : -INFINITY;
+            }
+        }
+#pragma unroll
+        for (int rt = 0; rt < 4; rt++) {
+            const float mt = fmaxf(fmaxf(sc[rt][0], sc[rt][1]), fmaxf(sc[rt][2], sc[rt][3]));
+            // the maximum and the rescale (by a power of two) only when some row's crosses an integer
+            if (__ballot(mt * c2 > m[rt]) != 0ull) { // wavefront-uniform
+                float2 b2 = both16(mt);
+                b2 = both32(fmaxf(b2.x, b2.y));
+                const float m_new = fmaxf(m[rt], ceilf(fmaxf(b2.x, b2.y) * c2));
+                const float f = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m[rt] - m_new);
+                lsum[rt] *= f;
+#pragma unroll
+                for (int dt = 0; dt < NK; dt++) o[rt][dt] *= f;
+                m[rt] = m_new;
+            }
+        }
+        half8v vv[NK]; // V beside itself: one 32-deep product takes p's hi and lo parts together
+#pragma unroll
+        for (int dt = 0; dt < NK; dt++) vv[dt] = join(vr[dt], vr[dt]);
+#pragma unroll
+        for (int rt = 0; rt < 4; rt++) {
+            const float m_ref = m[rt] == -INFINITY ? 0.0f : m[rt];
+            half4v ph, pl;
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const float pv = __builtin_amdgcn_exp2f(fmaf(sc[rt][v], c2, -m_ref));
+                ph[v] = (_Float16) pv;
+                pl[v] = (_Float16) fmaf((float) ph[v], -1.0f, pv);
+                lsum[rt] += pv;
+            }
+            const half8v pf = join(ph, pl);
+#pragma unroll
+            for (int dt = 0; dt < NK; dt++) o[rt][dt] = mfma32(vv[dt], pf, o[rt][dt]);
+        }
+        load_v(bn);
+    }
+    // the wavefronts' rows: out = sum_w o_w 2^(m_w - M), wavefronts in order, half of the dims at a time; then
+    // wavefront w finishes tile w / 2 and half of that half's dim tiles
+#pragma unroll
+    for (int rt = 0; rt < 4; rt++) {
+        float2 b2 = both16(lsum[rt]);
+        b2 = both32(b2.x + b2.y);
+        if (lq == 0) {
+            S.m[wave][16 * rt + lr] = m[rt];
+            S.l[wave][16 * rt + lr] = b2.x + b2.y;
+        }
+    }
+    constexpr int NH = NK / 2, NO = NH / 2; // dim tiles per half, per finishing wavefront
+    const int rt = wave >> 1, r = rb * 64 + 16 * rt + lr, t = min(r, rows - 1) / grp, h = g * grp + min(r, rows - 1) % grp;
+    float f[kAsWaves], M = -INFINITY, L = 0.0f;
+#pragma unroll
+    for (int half = 0; half < 2; half++) {
+        __syncthreads();
+#pragma unroll
+        for (int x = 0; x < 4; x++)
+#pragma unroll
+            for (int dt = 0; dt < NH; dt++) S.o[wave][x][dt][l] = o[x][half * NH + dt];
+        __syncthreads();
+        if (half == 0) {
+#pragma unroll
+            for (int x = 0; x < kAsWaves; x++) M = fmaxf(M, S.m[x][16 * rt + lr]);
+#pragma unroll
+            for (int x = 0; x < kAsWaves; x++) {
+                const float mx = S.m[x][16 * rt + lr];
+                f[x] = mx == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mx - M);
+                L += S.l[x][16 * rt + lr] * f[x];
+            }
+        }
+#pragma unroll
+        for (int d2 = 0; d2 < NO; d2++) {
+            const int dl = (wave & 1) * NO + d2, dt = half * NH + dl;
+            f32x4v y = {0, 0, 0, 0};
+#pragma unroll
+            for (int x = 0; x < kAsWaves; x++) y += S.o[x][rt][dl][l] * f[x];
+            if (r >= rows) continue;
+            // lane (row lr, quad lq) holds dims dt*16 + 4 lq .. +3 of its row
+            if (P.n_chunk == 1) {
+                const size_t oi = ((size_t) t * P.n_head + h) * HD + dt * 16 + 4 * lq;
+                const float4 z = make_float4(y[0] / L, y[1] / L, y[2] / L, y[3] / L);
+                *reinterpret_cast<float4 *>(P.out + oi) = z;
+                if (P.out16) *reinterpret_cast<uint2 *>(P.out16 + oi) = make_uint2(pack2(z.x, z.y), pack2(z.z, z.w));
+            } else {
+                float *pp = P.part + (((size_t) t * P.n_head + h) * P.n_chunk + c) * (HD + 4);
+                *reinterpret_cast<float4 *>(pp + 4 + dt * 16 + 4 * lq) = make_float4(y[0], y[1], y[2], y[3]);
+                if (dt == 0 && lq == 0) {
+                    pp[0] = M;
+                    pp[1] = L;
+                }
+            }
+        }
+    }
+}
+
 // Merges the chunks' partial rows of one (query head, token): out = sum_c o_c e^(m_c - M) / sum_c l_c e^(m_c - M).
 // Every load is issued before the first reduction: thread i takes chunk i's (m, l) (and chunks i + 256,
 // ... past 256 chunks), and hd / 4 threads per chunk hold the float4 slices of up to kCombRegs chunks
 // each in registers (chunks cl, cl + CL, ...; any further ones are read after the factors). Each
 // thread's slices are summed in ascending chunk order, then the CL thread sums in order.
+// BASE2: the partial rows of attn_split_kernel, whose maxima are exponents of 2 (integers, so the factors are exact).
 constexpr int kCombRegs = 16;
-template <int HD>
+template <int HD, bool BASE2>
 __global__ __launch_bounds__(kBlock) void attn_combine_kernel(AttnParams P) {
+    auto ex = [](float x) { return BASE2 ? __builtin_amdgcn_exp2f(x) : expf(x); };
     extern __shared__ float s_f[]; // [n_chunk] factors, then [kBlock / (hd / 4)][hd] sums
     __shared__ float s_red[kBlock / kWave];
     const int h = blockIdx.x, t = blockIdx.y, tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
@@ -1247,13 +1501,13 @@ __global__ __launch_bounds__(kBlock) void attn_combine_kernel(AttnParams P) {
     __syncthreads();
     float ls = 0.0f;
     if (tid < n) {
-        const float f = m0 == -INFINITY ? 0.0f : expf(m0 - M);
+        const float f = m0 == -INFINITY ? 0.0f : ex(m0 - M);
         s_f[tid] = f;
         ls += l0 * f;
     }
     for (int c = tid + kBlock; c < n; c += kBlock) {
         const float mc = pp[(size_t) c * stride];
-        const float f = mc == -INFINITY ? 0.0f : expf(mc - M);
+        const float f = mc == -INFINITY ? 0.0f : ex(mc - M);
         s_f[c] = f;
         ls += pp[(size_t) c * stride + 1] * f;
     }
@@ -1492,6 +1746,9 @@ hipError_t launch_rope(const RopeParams &P, hipStream_t st, const LaunchTiming *
     return launch(rope_kernel, dim3(P.T, P.n_head + 2 * P.n_kv), dim3(kWave), 0, st, tm, P);
 }
 
+// Launches of attn_split_kernel: many-token steps in 64-row blocks (head size 256 would need 128 KB of fragments a block).
+bool attn_in_split(const AttnParams &P) { return P.T >= kAttnSkipMinT && P.rb_rows == 64 && !P.rope_in && P.hd <= 128; }
+
 template <int HD>
 hipError_t launch_attn_hd(const AttnParams &P, hipStream_t st, const LaunchTiming *tm) {
     const dim3 grid(P.n_kv * P.n_chunk * P.n_rowblk), block(kAtBlock);
@@ -1506,8 +1763,14 @@ hipError_t launch_attn_hd(const AttnParams &P, hipStream_t st, const LaunchTimin
     // fragments per block)
     if constexpr (HD <= 128) {
         if (P.rb_rows == 64 && !P.rope_in) {
-            if (P.T >= kAttnSkipMinT) return launch(attn_rows_kernel<HD, true>, grid, block, 0, st, tm, P);
-            return launch(attn_rows_kernel<HD, false>, grid, block, 0, st, tm, P);
+            if (attn_in_split(P)) {
+                constexpr size_t lds = sizeof(AttnSplitLds<HD>);
+                static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_split_kernel<HD>),
+                                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
+                if (allowed != hipSuccess) return allowed;
+                return launch(attn_split_kernel<HD>, grid, dim3(kAsWaves * kWave), lds, st, tm, P);
+            }
+            return launch(attn_rows_kernel<HD>, grid, block, 0, st, tm, P);
         }
     }
     // steps of many tokens (prompts): the instantiation that skips passes with no cell of the sequence
@@ -1538,10 +1801,11 @@ hipError_t launch_attn_combine(const AttnParams &P, hipStream_t st, const Launch
     if (P.T == 0 || P.n_chunk == 1) return hipSuccess;
     const size_t lds = ((size_t) ((P.n_chunk + 3) & ~3) + (size_t) kBlock / (P.hd / 4) * P.hd) * sizeof(float);
     const dim3 grid(P.n_head, P.T), block(kBlock);
+    const bool base2 = attn_in_split(P);
     switch (P.hd) {
-    case 64: return launch(attn_combine_kernel<64>, grid, block, lds, st, tm, P);
-    case 128: return launch(attn_combine_kernel<128>, grid, block, lds, st, tm, P);
-    case 256: return launch(attn_combine_kernel<256>, grid, block, lds, st, tm, P);
+    case 64: return base2 ? launch(attn_combine_kernel<64, true>, grid, block, lds, st, tm, P) : launch(attn_combine_kernel<64, false>, grid, block, lds, st, tm, P);
+    case 128: return base2 ? launch(attn_combine_kernel<128, true>, grid, block, lds, st, tm, P) : launch(attn_combine_kernel<128, false>, grid, block, lds, st, tm, P);
+    case 256: return launch(attn_combine_kernel<256, false>, grid, block, lds, st, tm, P);
     default: return hipErrorInvalidValue;
     }
 }
