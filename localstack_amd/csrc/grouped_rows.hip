@@ -3,7 +3,7 @@
 //
 // Work item = up to 16 MT pairs of one expert (permute_kernel's list, grouped.hip; 16-row products rather than 32 because
 // a few hundred tokens leave each of 128 experts some 10 to 40 pairs, and products of rows past the last are wasted). A work-group stages the item's
-// quantized activation rows in LDS once, whole rows, and meets at one barrier; after that each of its four wavefronts
+// quantized activation rows in LDS once, whole rows, and meets at one barrier; after that each of its NW wavefronts
 // streams the weight rows of its own two 16-row tiles (gate and up of 16 rows, or 32 down rows) from memory straight
 // into registers, the next super-block requested before the current one is multiplied, and never waits for another
 // wavefront again. The pool layout already is the operand layout: of a 32-value block, lane (kg, r) = (lane / 16,
@@ -24,7 +24,7 @@
 // Bound: the expert bytes while an expert has a few pairs (64 tokens through a 30B-shaped Q2_K + Q3_K layer: 153 us for
 // 717 MB of unpacked weights), VALU work on the products past that. Against the GEMV kernels, which served these calls
 // before with dot products on the VALU and a work-group per expert however many pairs it had, on 30B-shaped layers on
-// MI355X: 512 tokens Q8_0 630 -> 207 us a layer, 203 tokens Q4_K + Q6_K 329 -> 132, 64 tokens Q2_K + Q3_K 200 -> 153.
+// MI355X: 512 tokens Q8_0 630 -> 200 us a layer, 203 tokens Q4_K + Q6_K 329 -> 132, 64 tokens Q2_K + Q3_K 200 -> 153.
 #include "device.h"
 #include "formats.h"
 #include "kernels.h"
@@ -41,13 +41,18 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) void lds_void;
 
-constexpr int kRThreads = 256;             // 4 wavefronts
 constexpr int kRXcds = 8;
 constexpr int kMagic = 0x4b400000;         // bits of 1.5 2^23
 constexpr float kMagicF = 12582912.0f;
 
 __device__ __forceinline__ i32x4 mfma8(uint2 a, uint2 b, i32x4 c) {
     return __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, a), __builtin_bit_cast(long, b), c, 0, 0, 0);
+}
+
+// v as a value of this place: what is derived from it is formed here and not ahead of time, held in registers.
+__device__ __forceinline__ unsigned here(unsigned v) {
+    asm volatile("" : "+v"(v));
+    return v;
 }
 
 // One 256-value super-block of a 16-row tile as the lane holds it: its share of the quants, and the rows' scales.
@@ -109,11 +114,11 @@ __host__ __device__ inline size_t r_lds(int CH, int K, unsigned char *base, RLds
 
 // Stages the item's n activation rows. Rows n .. CH - 1 keep stale bytes (their products are never stored), their
 // scales repeat row n - 1's.
-template <int WT, int CH>
+template <int WT, int CH, int NW>
 __device__ __forceinline__ void stage_rows(const GroupedParams &P, const RLds &L, int n) {
     const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int K = P.K, np = K / 16, nsb = K / 256;
-    for (int t = wave; t < n; t += 4) {
+    for (int t = wave; t < n; t += NW) {
         const int8_t *row = P.xqs + (size_t) __builtin_amdgcn_readfirstlane(L.src[t]) * K;
         for (int c0 = 0; c0 < np; c0 += kWave) {
             const int c = c0 + lane;
@@ -121,7 +126,7 @@ __device__ __forceinline__ void stage_rows(const GroupedParams &P, const RLds &L
         }
     }
     if constexpr (WT == kTypeQ8_0) {
-        for (int i = tid; i < CH * (K / 128); i += kRThreads) {
+        for (int i = tid; i < CH * (K / 128); i += NW * kWave) {
             const int t = i % CH, q4 = i / CH;
             const float4 v = *reinterpret_cast<const float4 *>(P.xd + (size_t) L.src[min(t, n - 1)] * (K / 32) + 4 * q4);
             L.dx[(4 * q4) * CH + t] = v.x;
@@ -130,13 +135,13 @@ __device__ __forceinline__ void stage_rows(const GroupedParams &P, const RLds &L
             L.dx[(4 * q4 + 3) * CH + t] = v.w;
         }
     } else {
-        for (int i = tid; i < CH * nsb; i += kRThreads) {
+        for (int i = tid; i < CH * nsb; i += NW * kWave) {
             const int t = i % CH, sb = i / CH;
             L.dx[sb * CH + t] = P.xd[(size_t) L.src[min(t, n - 1)] * (K / 32) + 8 * sb];
         }
     }
     if constexpr (WT == kTypeQ4_K) {
-        for (int i = tid; i < CH * nsb * 2; i += kRThreads) {
+        for (int i = tid; i < CH * nsb * 2; i += NW * kWave) {
             const int t = i % CH, hb = i / CH; // half super-block
             const uint4 v = *reinterpret_cast<const uint4 *>(P.xbh + (size_t) L.src[min(t, n - 1)] * (K / 32) + 4 * hb);
             *reinterpret_cast<uint4 *>(L.bh + ((hb / 2) * CH + t) * 8 + 4 * (hb & 1)) = v;
@@ -159,7 +164,7 @@ template <int WT, int MT, int CH>
 __device__ __forceinline__ void load_acts(Acts<WT, MT> &x, const RLds &L, int K, int sb, int b) {
     const unsigned lane = threadIdx.x % kWave, r = lane % 16, kg = lane / 16;
     // piece 2 b + kg / 2 of row r at slot (2 b + kg / 2) ^ r; b only flips bits 5-7 of the byte offset
-    const unsigned a0 = r * K + sb * 256 + (((kg >> 1) ^ r) * 16) + 8 * (kg & 1), zo = (unsigned) (L.z - L.a);
+    const unsigned a0 = here(r * K + (((kg >> 1) ^ r) * 16) + 8 * (kg & 1)) + sb * 256, zo = (unsigned) (L.z - L.a);
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
         const unsigned at = a0 + 16 * mt * K;
@@ -243,7 +248,8 @@ __device__ __forceinline__ void rows_products(const RLds &L, int K, const uint8_
                 i32x4 I[2][MT];
 #pragma unroll
                 for (int t = 0; t < 2; t++) {
-                    d[t] = h2f((b & 1) ? dw(h[t].h, b / 2) >> 16 : dw(h[t].h, b / 2));
+                    const unsigned d2 = here(dw(h[t].h, b / 2));
+                    d[t] = h2f((b & 1) ? d2 >> 16 : d2);
                     c[t] = -kMagicF * d[t];
 #pragma unroll
                     for (int mt = 0; mt < MT; mt++) I[t][mt] = mfma8(x.a[0][mt], q[t].q[b], magic);
@@ -390,17 +396,17 @@ __device__ __forceinline__ bool r_item(const GroupedParams &P, int n_rb, int4 &i
     return true;
 }
 
-// DOWN = false: wavefront w computes gate and up of rows rb * 64 + 16 w .. + 15 and stores silu(gate) * up.
-// DOWN = true: down rows rb * 128 + 32 w .. + 31, times the pair's router weight.
-template <int WT, bool MINS, int MT, bool DOWN>
-__global__ __launch_bounds__(kRThreads, MT == 1 ? 3 : 2) void rows_kernel(GroupedParams P) {
+// DOWN = false: wavefront w computes gate and up of rows 16 (rb NW + w) .. + 15 and stores silu(gate) * up.
+// DOWN = true: down rows 32 (rb NW + w) .. + 31, times the pair's router weight.
+template <int WT, bool MINS, int MT, bool DOWN, int NW>
+__global__ __launch_bounds__(NW *kWave, WT == kTypeKQ8 ? (NW == 8 ? 2 : 3) : 4) void rows_kernel(GroupedParams P) {
     constexpr int CH = 16 * MT, C = chunks_of(WT);
     extern __shared__ __align__(16) unsigned char smem[];
     RLds L;
     r_lds<WT>(CH, P.K, smem, &L);
     int4 it;
     int rb;
-    if (!r_item(P, P.rows / (DOWN ? 128 : 64), it, rb)) return;
+    if (!r_item(P, P.rows / (DOWN ? 32 * NW : 16 * NW), it, rb)) return;
     const int n = it.z, tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     if (tid < CH) {
         const int p = P.perm[it.y + min(tid, n - 1)];
@@ -408,11 +414,11 @@ __global__ __launch_bounds__(kRThreads, MT == 1 ? 3 : 2) void rows_kernel(Groupe
         L.src[tid] = p / P.row_div;
     }
     const size_t tb = (size_t) (P.K / 256) * (C * 256); // bytes of a 16-row block
-    const int row0 = DOWN ? rb * 128 + 32 * wave : rb * 64 + 16 * wave;
+    const int row0 = DOWN ? (rb * NW + wave) * 32 : (rb * NW + wave) * 16;
     const uint8_t *w0 = P.w0 + (size_t) it.x * P.stride0 + (size_t) (row0 / 16) * tb;
     const uint8_t *w1 = DOWN ? w0 + tb : P.w1 + (size_t) it.x * P.stride1 + (size_t) (row0 / 16) * tb;
     __syncthreads();
-    stage_rows<WT, CH>(P, L, n);
+    stage_rows<WT, CH, NW>(P, L, n);
     TileQ<WT> q[2];
     TileH<WT, MINS> h[2];
     load_h(h[0], w0);
@@ -424,46 +430,48 @@ __global__ __launch_bounds__(kRThreads, MT == 1 ? 3 : 2) void rows_kernel(Groupe
     }
     __syncthreads();
     const int kg = lane / 16, r = lane % 16;
-    auto store = [&](const auto &acc, auto mt_n) {
+    f32x4 acc[2][MT];
+    rows_products<WT, MINS, MT, CH>(L, P.K, w0, w1, q, h, acc);
 #pragma unroll
-        for (int mt = 0; mt < mt_n; mt++) {
+    for (int mt = 0; mt < MT; mt++) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int pos = 16 * mt + 4 * kg + i;
-                if (pos < n) {
-                    const int p = L.pair[pos];
-                    float *out = P.out + (size_t) p * P.rows + row0 + r;
-                    if constexpr (DOWN) {
-                        const float wt = P.weights[p];
-                        out[0] = acc[0][mt][i] * wt;
-                        out[16] = acc[1][mt][i] * wt;
-                    } else {
-                        const float gs = acc[0][mt][i], us = acc[1][mt][i];
-                        out[0] = (gs / (1.0f + expf(-gs))) * us;
-                    }
+        for (int i = 0; i < 4; i++) {
+            const int pos = 16 * mt + 4 * kg + i;
+            if (pos < n) {
+                const int p = L.pair[pos];
+                float *out = P.out + (size_t) p * P.rows + row0 + r;
+                if constexpr (DOWN) {
+                    const float wt = P.weights[p];
+                    out[0] = acc[0][mt][i] * wt;
+                    out[16] = acc[1][mt][i] * wt;
+                } else {
+                    const float gs = acc[0][mt][i], us = acc[1][mt][i];
+                    out[0] = (gs / (1.0f + expf(-gs))) * us;
                 }
             }
         }
-    };
-    if (MT > 1 && n <= 16) {
-        f32x4 acc[2][1];
-        rows_products<WT, MINS, 1, CH>(L, P.K, w0, w1, q, h, acc);
-        store(acc, std::integral_constant<int, 1>{});
-    } else {
-        f32x4 acc[2][MT];
-        rows_products<WT, MINS, MT, CH>(L, P.K, w0, w1, q, h, acc);
-        store(acc, std::integral_constant<int, MT>{});
     }
 }
 
-template <int WT, bool MINS, int MT, bool DOWN>
-hipError_t launch_rows_t(const GroupedParams &P, int max_items, hipStream_t st, const LaunchTiming *tm) {
+template <int WT, bool MINS, int MT, bool DOWN, int NW>
+hipError_t launch_rows_n(const GroupedParams &P, int max_items, hipStream_t st, const LaunchTiming *tm) {
     const size_t lds = r_lds<WT>(16 * MT, P.K, nullptr, nullptr);
-    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void *>(&rows_kernel<WT, MINS, MT, DOWN>),
+    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void *>(&rows_kernel<WT, MINS, MT, DOWN, NW>),
                                                           hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     if (allowed != hipSuccess) return allowed;
     const int per = (max_items + kRXcds - 1) / kRXcds;
-    return launch(rows_kernel<WT, MINS, MT, DOWN>, dim3(kRXcds * per * (P.rows / (DOWN ? 128 : 64))), dim3(kRThreads), lds, st, tm, P);
+    return launch(rows_kernel<WT, MINS, MT, DOWN, NW>, dim3(kRXcds * per * (P.rows / (DOWN ? 32 * NW : 16 * NW))), dim3(NW * kWave), lds, st, tm, P);
+}
+// Gate / up work-groups take 8 wavefronts (128 rows) where the staged rows fill 64 KB or more, so that the two
+// work-groups a CU holds then are 16 wavefronts: 30B-shaped Q8_0 layer, 32-pair items, us with 4 / 8: 300 Zipf-routed
+// tokens 145 / 129, 512 194 / 181, 512 evenly routed 218 / 220; 235B shape, 16-pair Q4_K items, 64 tokens 315 / 295.
+// Below that 4 are faster (more work-groups overlap their starts: 64 tokens of Q2_K + Q3_K 159 / 186), and so they are
+// for down, whose rows are short (512 tokens Q8_0 214 / 244).
+template <int WT, bool MINS, int MT, bool DOWN>
+hipError_t launch_rows_t(const GroupedParams &P, int max_items, hipStream_t st, const LaunchTiming *tm) {
+    if constexpr (!DOWN)
+        if (16 * MT * P.K >= 64 * 1024 && P.rows % 128 == 0) return launch_rows_n<WT, MINS, MT, false, 8>(P, max_items, st, tm);
+    return launch_rows_n<WT, MINS, MT, DOWN, 4>(P, max_items, st, tm);
 }
 
 template <bool DOWN>
