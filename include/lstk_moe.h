@@ -165,9 +165,9 @@ int lstk_moe_route(lstk_pool *pool, int layer, const float *d_hnorm, int n_token
  * the weight type (Q8_0 for Q8_0, Q8_K for Q4_K), and so is the SwiGLU output before down.
  * d_slots holds slot numbers from lstk_pool_acquire (streaming) or expert ids (resident).
  * d_out may alias d_resid.
- * From 32 tokens on (49 with Q4_K gate, up and down; LSTK_GROUPED_MIN_TOKENS in the environment overrides the
- * threshold) the call takes the grouped path: a stable permutation of the pairs by expert, then expert products
- * on the matrix cores over chunks of 16 or 32 pairs. */
+ * From some tokens on (9 with Q4_K experts, up to 32 by format and expert size; LSTK_GROUPED_MIN_TOKENS in the
+ * environment overrides the threshold) the call takes the grouped path: a stable permutation of the pairs by
+ * expert, then expert products on the matrix cores over chunks of 16 or 32 pairs. */
 int lstk_moe_ffn(lstk_pool *pool, int layer, const float *d_hnorm, const int32_t *d_slots, const float *d_weights,
                  const float *d_resid, float *d_out, int n_tokens, lstk_stream_t stream);
 
@@ -185,10 +185,10 @@ int lstk_moe_block(lstk_pool *pool, int layer, const float *d_hnorm, const void 
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). The call's
  * scratch (quantized activations, router logits, SwiGLU rows, per-pair outputs) comes from a fixed
  * array of LSTK_NOALLOC_SCRATCH_BYTES in the library, one copy per device, held until the process
- * ends; the call allocates nothing and creates no events. Same arguments, kernels and results as
- * lstk_moe_block, except that it never takes the fused or the grouped (matrix-core prefill) path and
- * keeps no stage timing. Fails with LSTK_E_INVALID when n_tokens needs more scratch than the array
- * holds: n_tokens * (n_embd * (1.25 + 4 k) + 4 E + 4 k n_ff_exp) bytes, each part rounded up to 256
+ * ends (a call of many tokens also uses the pool's own work list and quantized SwiGLU rows, laid out at
+ * creation); the call allocates nothing and creates no events. Same arguments, kernels and results as
+ * lstk_moe_block, except that it never takes the fused path and keeps no stage timing. Fails with
+ * LSTK_E_INVALID when n_tokens needs more scratch than the array holds: n_tokens * (n_embd * (1.25 + 4 k) + 4 E + 4 k n_ff_exp) bytes, each part rounded up to 256
  * (up to 180 tokens at the 30B-A3B shape, 90 at the 235B-A22B shape; n_batch of the pool still
  * applies). Every call on a device shares that device's array, which keeps the last call's contents:
  * calls that overlap on one device race, whatever pool or stream they use. */

@@ -833,19 +833,27 @@ int check_call(lstk_pool *P, int layer, int T) {
     return LSTK_OK;
 }
 
-// The matrix-core path of many-token calls. A call takes it from T tokens on (LSTK_GROUPED_MIN_TOKENS overrides):
-// 32 with Q8_0 or KQ8 experts, 49 with Q4_K gate, up and down. Measured on one 30B-shaped layer, GEMV path against this
-// one, us a layer with even / Zipf(1.1) routing: Q8_0 24 tokens 101 / 112, 32 tokens 118 / 126 and 114 / 59, 48 tokens
-// 147 / 140; Q2_K + Q3_K 17 tokens 107 / 112, 32 tokens 144 / 136; Q4_K + Q6_K 32 tokens 110 / 100; Q4_K 50 tokens
-// 127 / 94 and 152 / 57 (up to 48 Q4_K tokens stay where lstk_moe_block_noalloc is bit-identical to lstk_moe_block).
-constexpr int kGroupedMinTokens = 32, kGroupedMinTokensQ4K = 49;
+// The matrix-core path of many-token calls: from how many tokens on a call takes it (LSTK_GROUPED_MIN_TOKENS overrides).
+// It costs two launches more than the GEMV path (permute, SwiGLU quantization) and wins where experts have several
+// pairs, which skewed routing brings early. Measured on one layer, GEMV path against this one, us:
+//   Q4_K gate, up and down: 30B shape 9 tokens 51 / 50 evenly routed and 45 / 40 Zipf(1.1)-routed, 12 61 / 56 and 53 / 40, 24
+//     80 / 68 and 87 / 43, 40 114 / 91; 235B shape 12 218 / 180.
+//   Q4_K gate and up, another k-quant down: 12 70 / 64, 17 83 / 75 and 73 / 44.
+//   KQ8 gate and up (Q2_K + Q3_K): 12 89 / 94 and 80 / 51, 17 107 / 112 and 106 / 55, 24 125 / 123 and 135 / 54.
+//   Q8_0: 24 101 / 112 and 86 / 61, 32 118 / 126 and 114 / 59, 48 147 / 140.
+// Experts below a million weights (the tiny shapes) are cheap either way, so their calls keep the fewer launches up to
+// 31 tokens (h 256, f 512, 8 experts, Q8_0: 17 tokens 28 / 35, 32 40 / 34).
+int grouped_from(const Shard &s, int h, int f) {
+    if ((long) 3 * h * f < 1000000 || s.tg == lstk::kTypeQ8_0) return 32;
+    if (s.tg != lstk::kTypeQ4_K) return 17;
+    return s.td == lstk::kTypeQ4_K ? 9 : s.td == lstk::kTypeQ8_0 ? 32 : 12;
+}
 bool use_grouped(lstk_pool *P, const Shard &s, int T) {
     if (P->grouped_min_tokens == 0) {
         const char *env = std::getenv("LSTK_GROUPED_MIN_TOKENS");
         P->grouped_min_tokens = env ? std::max(1, std::atoi(env)) : -1;
     }
-    const bool q4k = s.tg == lstk::kTypeQ4_K && s.td == lstk::kTypeQ4_K;
-    const int from = P->grouped_min_tokens > 0 ? P->grouped_min_tokens : q4k ? kGroupedMinTokensQ4K : kGroupedMinTokens;
+    const int from = P->grouped_min_tokens > 0 ? P->grouped_min_tokens : grouped_from(s, P->dims.n_embd, P->dims.n_ff_exp);
     return T >= from && lstk::grouped_supported(s.tu, s.tg, s.td, P->dims.n_embd, P->dims.n_ff_exp, (int) s.n_slots);
 }
 
@@ -864,67 +872,6 @@ GroupedPlan grouped_plan(const Shard &s, int np, int n_expert) {
     if (s.tg == lstk::kTypeQ4_K && s.td == lstk::kTypeQ4_K && np > 14 * n_expert) return {false, lstk::kGroupedChunk};
     const bool q8 = s.tg == lstk::kTypeQ8_0 && s.td == lstk::kTypeQ8_0;
     return {true, q8 && np > 12 * n_expert ? 32 : 16};
-}
-
-// permute -> gate_up (MFMA, SwiGLU) -> Q8_0 / Q8_K of the SwiGLU rows -> down (MFMA, router weight) ->
-// combine + residual. bins: expert ids (resident) or slots (streaming), [T][k].
-int run_grouped(lstk_pool *P, const Shard &s, const int32_t *bins, const float *d_weights, const float *d_resid,
-                float *d_out, int T, hipStream_t st) {
-    const lstk_moe_dims &d = P->dims;
-    const int k = d.n_expert_used, np = T * k, h = d.n_embd, f = d.n_ff_exp;
-    const auto [rows, chunk] = grouped_plan(s, np, d.n_expert);
-    const int max_items = lstk::grouped_max_items(np, (int) s.n_slots, chunk);
-    lstk::PermuteParams pp{bins, np, (int) s.n_slots, chunk, P->counts, P->offsets, P->perm,
-                           P->items, P->n_items, P->err, s.tg == lstk::kTypeQ4_K && s.td == lstk::kTypeQ4_K ? 0 : T};
-    hipError_t e = timed(P, 0, [&](const lstk::LaunchTiming *tm) { return lstk::launch_permute(pp, st, tm); });
-    if (e != hipSuccess) return hip_fail(e, "permute launch");
-    lstk::GroupedParams gu{};
-    gu.items = P->items;
-    gu.n_items = P->n_items;
-    gu.perm = P->perm;
-    gu.k = k;
-    gu.w0 = s.d_gate;
-    gu.w1 = s.d_up;
-    gu.stride0 = s.gate_bytes;
-    gu.stride1 = s.up_bytes;
-    gu.rows = f;
-    gu.K = h;
-    gu.xqs = P->xq.qs;
-    gu.xd = P->xq.d;
-    gu.xbh = P->xq.bh;
-    gu.row_div = k;
-    gu.out = P->act;
-    gu.type = s.tg;
-    gu.chunk = chunk;
-    e = timed(P, 1, [&, rows = rows](const lstk::LaunchTiming *tm) {
-        return rows ? lstk::launch_gate_up_rows(gu, max_items, st, tm) : lstk::launch_gate_up_grouped(gu, max_items, st, tm);
-    });
-    if (e != hipSuccess) return hip_fail(e, "gate_up launch");
-    e = timed(P, 2, [&](const lstk::LaunchTiming *tm) { return lstk::launch_act_quant(P->act, f, np, s.td, P->aq, st, tm); });
-    if (e != hipSuccess) return hip_fail(e, "act quant launch");
-    lstk::GroupedParams dn = gu;
-    dn.w0 = s.d_down;
-    dn.w1 = nullptr;
-    dn.stride0 = s.down_bytes;
-    dn.stride1 = 0;
-    dn.rows = h;
-    dn.K = f;
-    dn.xqs = P->aq.qs;
-    dn.xd = P->aq.d;
-    dn.xbh = P->aq.bh;
-    dn.row_div = 1;
-    dn.weights = d_weights;
-    dn.out = P->Y;
-    dn.type = s.td;
-    e = timed(P, 2, [&, rows = rows](const lstk::LaunchTiming *tm) {
-        return rows ? lstk::launch_down_rows(dn, max_items, st, tm) : lstk::launch_down_grouped(dn, max_items, st, tm);
-    });
-    if (e != hipSuccess) return hip_fail(e, "down launch");
-    if (P->defer_combine) return LSTK_OK;
-    lstk::CombineParams cp{P->Y, d_resid, d_out, T, k, h};
-    e = timed(P, 3, [&](const lstk::LaunchTiming *tm) { return lstk::launch_combine(cp, st, tm); });
-    if (e != hipSuccess) return hip_fail(e, "combine launch");
-    return LSTK_OK;
 }
 
 // The fused single-token path (one launch per block) is opt-in: LSTK_FUSED_DECODE=1 at pool creation.
@@ -994,7 +941,7 @@ struct NormIn {
     float eps;
 };
 
-// Per-call device scratch of the GEMV path: the pool's own (sized for n_batch at creation) or a layout in
+// Per-call device scratch of both paths: the pool's own (sized for n_batch at creation) or a layout in
 // the fixed array of lstk_moe_block_noalloc.
 struct CallScratch {
     lstk::ActBuf xq;
@@ -1024,9 +971,74 @@ size_t call_scratch_layout(const lstk_moe_dims &d, int T, uint8_t *base, CallScr
     return off;
 }
 
-// fixed != null (lstk_moe_block_noalloc): the scratch comes from the fixed array, and the call takes
-// neither the fused nor the grouped path (their counters and work lists live in the pool's scratch)
-// nor the stage timing (which creates events).
+// permute -> gate_up (MFMA, SwiGLU) -> Q8_0 / Q8_K of the SwiGLU rows -> down (MFMA, router weight) ->
+// combine + residual. bins: expert ids (resident) or slots (streaming), [T][k].
+// fixed: the activations, SwiGLU rows and outputs are in the fixed array of lstk_moe_block_noalloc, no stage timing.
+int run_grouped(lstk_pool *P, const Shard &s, const CallScratch &sc, bool fixed, const int32_t *bins, const float *d_weights,
+                const float *d_resid, float *d_out, int T, hipStream_t st) {
+    auto timed = [&](lstk_pool *pool, int stage, auto &&launch) -> hipError_t {
+        return fixed ? launch(nullptr) : ::timed(pool, stage, launch);
+    };
+    const lstk_moe_dims &d = P->dims;
+    const int k = d.n_expert_used, np = T * k, h = d.n_embd, f = d.n_ff_exp;
+    const auto [rows, chunk] = grouped_plan(s, np, d.n_expert);
+    const int max_items = lstk::grouped_max_items(np, (int) s.n_slots, chunk);
+    lstk::PermuteParams pp{bins, np, (int) s.n_slots, chunk, P->counts, P->offsets, P->perm,
+                           P->items, P->n_items, P->err, T < 64 || s.tg != lstk::kTypeQ4_K || s.td != lstk::kTypeQ4_K ? T : 0};
+    hipError_t e = timed(P, 0, [&](const lstk::LaunchTiming *tm) { return lstk::launch_permute(pp, st, tm); });
+    if (e != hipSuccess) return hip_fail(e, "permute launch");
+    lstk::GroupedParams gu{};
+    gu.items = P->items;
+    gu.n_items = P->n_items;
+    gu.perm = P->perm;
+    gu.k = k;
+    gu.w0 = s.d_gate;
+    gu.w1 = s.d_up;
+    gu.stride0 = s.gate_bytes;
+    gu.stride1 = s.up_bytes;
+    gu.rows = f;
+    gu.K = h;
+    gu.xqs = sc.xq.qs;
+    gu.xd = sc.xq.d;
+    gu.xbh = P->xq.bh;
+    gu.row_div = k;
+    gu.out = sc.act;
+    gu.type = s.tg;
+    gu.chunk = chunk;
+    e = timed(P, 1, [&, rows = rows](const lstk::LaunchTiming *tm) {
+        return rows ? lstk::launch_gate_up_rows(gu, max_items, st, tm) : lstk::launch_gate_up_grouped(gu, max_items, st, tm);
+    });
+    if (e != hipSuccess) return hip_fail(e, "gate_up launch");
+    e = timed(P, 2, [&](const lstk::LaunchTiming *tm) { return lstk::launch_act_quant(sc.act, f, np, s.td, P->aq, st, tm); });
+    if (e != hipSuccess) return hip_fail(e, "act quant launch");
+    lstk::GroupedParams dn = gu;
+    dn.w0 = s.d_down;
+    dn.w1 = nullptr;
+    dn.stride0 = s.down_bytes;
+    dn.stride1 = 0;
+    dn.rows = h;
+    dn.K = f;
+    dn.xqs = P->aq.qs;
+    dn.xd = P->aq.d;
+    dn.xbh = P->aq.bh;
+    dn.row_div = 1;
+    dn.weights = d_weights;
+    dn.out = sc.Y;
+    dn.type = s.td;
+    e = timed(P, 2, [&, rows = rows](const lstk::LaunchTiming *tm) {
+        return rows ? lstk::launch_down_rows(dn, max_items, st, tm) : lstk::launch_down_grouped(dn, max_items, st, tm);
+    });
+    if (e != hipSuccess) return hip_fail(e, "down launch");
+    if (P->defer_combine && !fixed) return LSTK_OK;
+    lstk::CombineParams cp{sc.Y, d_resid, d_out, T, k, h};
+    e = timed(P, 3, [&](const lstk::LaunchTiming *tm) { return lstk::launch_combine(cp, st, tm); });
+    if (e != hipSuccess) return hip_fail(e, "combine launch");
+    return LSTK_OK;
+}
+
+// fixed != null (lstk_moe_block_noalloc): the scratch comes from the fixed array (a many-token call's work list and its
+// quantized SwiGLU rows from the pool's, laid out for n_batch at creation), and the call takes neither the fused path nor
+// the stage timing (which creates events).
 int run_block(lstk_pool *P, int layer, int mode, const float *d_hnorm, const void *d_gate_inp, int gate_type,
               const int32_t *d_slots, int32_t *d_ids, float *d_weights, const float *d_resid, float *d_out, int T,
               hipStream_t st, const NormIn *norm = nullptr, const CallScratch *fixed = nullptr) {
@@ -1056,8 +1068,8 @@ int run_block(lstk_pool *P, int layer, int mode, const float *d_hnorm, const voi
     rp.logits = sc.logits;
     rp.qtype = s.tu;
     rp.xq = sc.xq;
-    const bool grouped = !fixed && use_grouped(P, s, T);
-    if (!grouped) rp.xq.bh = nullptr; // only the grouped kernels read the split group sums
+    const bool grouped = use_grouped(P, s, T);
+    rp.xq.bh = grouped ? P->xq.bh : nullptr; // only the grouped kernels read the split group sums
     hipError_t e = timed(P, 0, [&](const lstk::LaunchTiming *tm) { return lstk::launch_route(rp, st, tm); });
     if (e != hipSuccess) return hip_fail(e, "route launch");
     const bool fused_topk = mode == 1 && T <= lstk::decode_route_max_tokens();
@@ -1067,7 +1079,7 @@ int run_block(lstk_pool *P, int layer, int mode, const float *d_hnorm, const voi
         if (e != hipSuccess) return hip_fail(e, "topk launch");
     }
     if (grouped)
-        return run_grouped(P, s, mode == 1 ? d_ids : d_slots, d_weights, d_resid, d_out, T, st);
+        return run_grouped(P, s, sc, fixed != nullptr, mode == 1 ? d_ids : d_slots, d_weights, d_resid, d_out, T, st);
     lstk::GroupParams gp{};
     gp.T = T;
     gp.k = k;
