@@ -188,7 +188,8 @@ int lstk_moe_block(lstk_pool *pool, int layer, const float *d_hnorm, const void 
  * ends (a call of many tokens also uses the pool's own work list and quantized SwiGLU rows, laid out at
  * creation); the call allocates nothing and creates no events. Same arguments, kernels and results as
  * lstk_moe_block, except that it never takes the fused path and keeps no stage timing. Fails with
- * LSTK_E_INVALID when n_tokens needs more scratch than the array holds: n_tokens * (n_embd * (1.25 + 4 k) + 4 E + 4 k n_ff_exp) bytes, each part rounded up to 256
+ * LSTK_E_INVALID when n_tokens needs more scratch than the array holds:
+ * n_tokens * (n_embd * (1.25 + 4 k) + 4 E + 4 k n_ff_exp) bytes, each part rounded up to 256
  * (up to 180 tokens at the 30B-A3B shape, 90 at the 235B-A22B shape; n_batch of the pool still
  * applies). Every call on a device shares that device's array, which keeps the last call's contents:
  * calls that overlap on one device race, whatever pool or stream they use. */

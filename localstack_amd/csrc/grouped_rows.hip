@@ -24,7 +24,8 @@
 // Bound: the expert bytes while an expert has a few pairs (64 tokens through a 30B-shaped Q2_K + Q3_K layer: 153 us for
 // 717 MB of unpacked weights), VALU work on the products past that. Against the GEMV kernels, which served these calls
 // before with dot products on the VALU and a work-group per expert however many pairs it had, on 30B-shaped layers on
-// MI355X: 512 tokens Q8_0 630 -> 200 us a layer, 203 tokens Q4_K + Q6_K 329 -> 132, 64 tokens Q2_K + Q3_K 200 -> 153.
+// MI355X: 512 tokens Q8_0 630 -> 200 us a layer, 203 tokens Q4_K + Q6_K 329 -> 132, 64 tokens Q2_K + Q3_K 200 -> 153 (-> 134 with
+// the weights' non-temporal loads of calls whose experts mostly have one item, GroupedParams::once).
 #include "device.h"
 #include "formats.h"
 #include "kernels.h"
@@ -67,21 +68,29 @@ struct TileH {
     float2 d[WT == kTypeKQ8 ? 1 : 0];                    // KQ8: d, dmin
 };
 
+// A weight load; NT: with the non-temporal hint (load_weights, device.h).
+template <bool NT, typename T>
+__device__ __forceinline__ T load_w(const uint8_t *p) {
+    typedef unsigned uv __attribute__((ext_vector_type(sizeof(T) / 4)));
+    const uv *q = reinterpret_cast<const uv *>(p);
+    return __builtin_bit_cast(T, NT ? __builtin_nontemporal_load(q) : *q);
+}
+
 // p: super-block of the tile (wavefront-uniform).
-template <int WT>
+template <int WT, bool NT>
 __device__ __forceinline__ uint2 load_q(const uint8_t *p, int b) {
     const unsigned lane = threadIdx.x % kWave, r = lane % 16, kg = lane / 16;
-    return *reinterpret_cast<const uint2 *>(p + ((WT == kTypeKQ8 ? 3 : 1) + (kg >> 1)) * 256 + r * 16 + 8 * (kg & 1) + 512 * b);
+    return load_w<NT, uint2>(p + ((WT == kTypeKQ8 ? 3 : 1) + (kg >> 1)) * 256 + r * 16 + 8 * (kg & 1) + 512 * b);
 }
-template <int WT, bool MINS>
+template <int WT, bool MINS, bool NT>
 __device__ __forceinline__ void load_h(TileH<WT, MINS> &t, const uint8_t *p) {
     const unsigned o = (threadIdx.x % 16) * 16;
     if constexpr (WT == kTypeKQ8) {
-        t.d[0] = *reinterpret_cast<const float2 *>(p + o);
-        t.h = *reinterpret_cast<const uint4 *>(p + o + 256);
-        if constexpr (MINS) t.m[0] = *reinterpret_cast<const uint4 *>(p + o + 512);
+        t.d[0] = load_w<NT, float2>(p + o);
+        t.h = load_w<NT, uint4>(p + o + 256);
+        if constexpr (MINS) t.m[0] = load_w<NT, uint4>(p + o + 512);
     } else {
-        t.h = *reinterpret_cast<const uint4 *>(p + o);
+        t.h = load_w<NT, uint4>(p + o);
     }
 }
 
@@ -202,7 +211,7 @@ __device__ __forceinline__ int sext_byte(unsigned v, int i) {
 // 16 mt + 4 (lane / 16) + i of the item, row lane % 16 of the tile. q / h hold super-block 0. A block's quants are
 // requested for the next super-block as soon as they have been multiplied, into the same registers, so every load
 // has a super-block's products to arrive in and no second copy of the tile is held.
-template <int WT, bool MINS, int MT, int CH>
+template <int WT, bool MINS, int MT, int CH, bool NT>
 __device__ __forceinline__ void rows_products(const RLds &L, int K, const uint8_t *w0, const uint8_t *w1, TileQ<WT> (&q)[2],
                                               TileH<WT, MINS> (&h)[2], f32x4 (&acc)[2][MT]) {
     constexpr int C = chunks_of(WT);
@@ -222,7 +231,7 @@ __device__ __forceinline__ void rows_products(const RLds &L, int K, const uint8_
 #pragma unroll
         for (int t = 0; t < 2; t++) {
             wp[t] += C * 256;
-            if constexpr (more) load_h(nh[t], wp[t]);
+            if constexpr (more) load_h<WT, MINS, NT>(nh[t], wp[t]);
         }
         i32x4 isum[2][WT == kTypeQ8_0 ? 0 : MT], imin[2][WT == kTypeKQ8 && MINS ? MT : 0];
         unsigned sc[2][2]; // Q4_K: the 6-bit scales, one per byte (sub-blocks 0-3 and 4-7)
@@ -322,7 +331,7 @@ __device__ __forceinline__ void rows_products(const RLds &L, int K, const uint8_
 #pragma unroll
                     for (int t = 0; t < 2; t++) {
                         const int bq = WT == kTypeQ4_K ? b / 2 : b;
-                        q[t].q[bq] = load_q<WT>(wp[t], bq);
+                        q[t].q[bq] = load_q<WT, NT>(wp[t], bq);
                     }
                 }
             }
@@ -398,7 +407,7 @@ __device__ __forceinline__ bool r_item(const GroupedParams &P, int n_rb, int4 &i
 
 // DOWN = false: wavefront w computes gate and up of rows 16 (rb NW + w) .. + 15 and stores silu(gate) * up.
 // DOWN = true: down rows 32 (rb NW + w) .. + 31, times the pair's router weight.
-template <int WT, bool MINS, int MT, bool DOWN, int NW>
+template <int WT, bool MINS, int MT, bool DOWN, int NW, bool NT>
 __global__ __launch_bounds__(NW *kWave, WT == kTypeKQ8 ? (NW == 8 ? 2 : 3) : 4) void rows_kernel(GroupedParams P) {
     constexpr int CH = 16 * MT, C = chunks_of(WT);
     extern __shared__ __align__(16) unsigned char smem[];
@@ -421,17 +430,17 @@ __global__ __launch_bounds__(NW *kWave, WT == kTypeKQ8 ? (NW == 8 ? 2 : 3) : 4) 
     stage_rows<WT, CH, NW>(P, L, n);
     TileQ<WT> q[2];
     TileH<WT, MINS> h[2];
-    load_h(h[0], w0);
-    load_h(h[1], w1);
+    load_h<WT, MINS, NT>(h[0], w0);
+    load_h<WT, MINS, NT>(h[1], w1);
 #pragma unroll
     for (int b = 0; b < (WT == kTypeQ4_K ? 4 : 8); b++) {
-        q[0].q[b] = load_q<WT>(w0, b);
-        q[1].q[b] = load_q<WT>(w1, b);
+        q[0].q[b] = load_q<WT, NT>(w0, b);
+        q[1].q[b] = load_q<WT, NT>(w1, b);
     }
     __syncthreads();
     const int kg = lane / 16, r = lane % 16;
     f32x4 acc[2][MT];
-    rows_products<WT, MINS, MT, CH>(L, P.K, w0, w1, q, h, acc);
+    rows_products<WT, MINS, MT, CH, NT>(L, P.K, w0, w1, q, h, acc);
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
 #pragma unroll
@@ -453,25 +462,31 @@ __global__ __launch_bounds__(NW *kWave, WT == kTypeKQ8 ? (NW == 8 ? 2 : 3) : 4) 
     }
 }
 
-template <int WT, bool MINS, int MT, bool DOWN, int NW>
+template <int WT, bool MINS, int MT, bool DOWN, int NW, bool NT>
 hipError_t launch_rows_n(const GroupedParams &P, int max_items, hipStream_t st, const LaunchTiming *tm) {
     const size_t lds = r_lds<WT>(16 * MT, P.K, nullptr, nullptr);
-    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void *>(&rows_kernel<WT, MINS, MT, DOWN, NW>),
+    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void *>(&rows_kernel<WT, MINS, MT, DOWN, NW, NT>),
                                                           hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     if (allowed != hipSuccess) return allowed;
     const int per = (max_items + kRXcds - 1) / kRXcds;
-    return launch(rows_kernel<WT, MINS, MT, DOWN, NW>, dim3(kRXcds * per * (P.rows / (DOWN ? 32 * NW : 16 * NW))), dim3(NW * kWave), lds, st, tm, P);
+    return launch(rows_kernel<WT, MINS, MT, DOWN, NW, NT>, dim3(kRXcds * per * (P.rows / (DOWN ? 32 * NW : 16 * NW))), dim3(NW * kWave), lds, st, tm, P);
 }
 // Gate / up work-groups take 8 wavefronts (128 rows) where the staged rows fill 64 KB or more, so that the two
 // work-groups a CU holds then are 16 wavefronts: 30B-shaped Q8_0 layer, 32-pair items, us with 4 / 8: 300 Zipf-routed
 // tokens 145 / 129, 512 194 / 181, 512 evenly routed 218 / 220; 235B shape, 16-pair Q4_K items, 64 tokens 315 / 295.
 // Below that 4 are faster (more work-groups overlap their starts: 64 tokens of Q2_K + Q3_K 159 / 186), and so they are
 // for down, whose rows are short (512 tokens Q8_0 214 / 244).
+template <int WT, bool MINS, int MT, bool DOWN, bool NT>
+hipError_t launch_rows_w(const GroupedParams &P, int max_items, hipStream_t st, const LaunchTiming *tm) {
+    if constexpr (!DOWN)
+        if (16 * MT * P.K >= 64 * 1024 && P.rows % 128 == 0) return launch_rows_n<WT, MINS, MT, false, 8, NT>(P, max_items, st, tm);
+    return launch_rows_n<WT, MINS, MT, DOWN, 4, NT>(P, max_items, st, tm);
+}
 template <int WT, bool MINS, int MT, bool DOWN>
 hipError_t launch_rows_t(const GroupedParams &P, int max_items, hipStream_t st, const LaunchTiming *tm) {
-    if constexpr (!DOWN)
-        if (16 * MT * P.K >= 64 * 1024 && P.rows % 128 == 0) return launch_rows_n<WT, MINS, MT, false, 8>(P, max_items, st, tm);
-    return launch_rows_n<WT, MINS, MT, DOWN, 4>(P, max_items, st, tm);
+    if constexpr (MT == 1)
+        if (P.once) return launch_rows_w<WT, MINS, MT, DOWN, true>(P, max_items, st, tm);
+    return launch_rows_w<WT, MINS, MT, DOWN, false>(P, max_items, st, tm);
 }
 
 template <bool DOWN>

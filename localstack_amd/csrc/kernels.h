@@ -148,6 +148,7 @@ struct GroupedParams {
     float *out;
     int type;                // ggml type of the weights
     int chunk;               // pairs per work item
+    bool once;               // 16-pair items: most experts have one item, so their weights carry the non-temporal hint
 };
 
 // The whole MoE block of one token in one launch (fused.hip). Work-groups [0, nB) each compute one

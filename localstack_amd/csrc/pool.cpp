@@ -864,14 +864,19 @@ bool use_grouped(lstk_pool *P, const Shard &s, int T) {
 // chunk: 16 pairs (one matrix-core tile, 36 KB of LDS at h 2048) or, for Q8_0 past 12 pairs per expert, 32 (us: 200
 //   tokens 165 / 165, 256 181 / 174, 400 214 / 199, 300 Zipf-routed 153 / 137). KQ8 stays at 16: its second tile takes
 //   the kernel past 200 VGPRs (203 tokens 135 / 200).
+// once: up to 4 pairs per expert on average most experts have one item, whose weights are read once: with the
+//   non-temporal hint they do not displace what is read again (us without / with: 64 evenly routed tokens of Q4_K 99 / 87,
+//   Q8_0 144 / 127, Q2_K + Q3_K 158 / 138; Zipf-routed, where hot experts' items share weights in L2, 58 / 61, 78 / 85,
+//   75 / 82; past 4 pairs that side loses more: 128 tokens of Q8_0 158 / 139 and 94 / 105).
 struct GroupedPlan {
     bool rows;
     int chunk;
+    bool once;
 };
 GroupedPlan grouped_plan(const Shard &s, int np, int n_expert) {
-    if (s.tg == lstk::kTypeQ4_K && s.td == lstk::kTypeQ4_K && np > 14 * n_expert) return {false, lstk::kGroupedChunk};
+    if (s.tg == lstk::kTypeQ4_K && s.td == lstk::kTypeQ4_K && np > 14 * n_expert) return {false, lstk::kGroupedChunk, false};
     const bool q8 = s.tg == lstk::kTypeQ8_0 && s.td == lstk::kTypeQ8_0;
-    return {true, q8 && np > 12 * n_expert ? 32 : 16};
+    return {true, q8 && np > 12 * n_expert ? 32 : 16, np <= 4 * n_expert};
 }
 
 // The fused single-token path (one launch per block) is opt-in: LSTK_FUSED_DECODE=1 at pool creation.
@@ -981,7 +986,7 @@ int run_grouped(lstk_pool *P, const Shard &s, const CallScratch &sc, bool fixed,
     };
     const lstk_moe_dims &d = P->dims;
     const int k = d.n_expert_used, np = T * k, h = d.n_embd, f = d.n_ff_exp;
-    const auto [rows, chunk] = grouped_plan(s, np, d.n_expert);
+    const auto [rows, chunk, once] = grouped_plan(s, np, d.n_expert);
     const int max_items = lstk::grouped_max_items(np, (int) s.n_slots, chunk);
     lstk::PermuteParams pp{bins, np, (int) s.n_slots, chunk, P->counts, P->offsets, P->perm,
                            P->items, P->n_items, P->err, T < 64 || s.tg != lstk::kTypeQ4_K || s.td != lstk::kTypeQ4_K ? T : 0};
@@ -1005,6 +1010,7 @@ int run_grouped(lstk_pool *P, const Shard &s, const CallScratch &sc, bool fixed,
     gu.out = sc.act;
     gu.type = s.tg;
     gu.chunk = chunk;
+    gu.once = once;
     e = timed(P, 1, [&, rows = rows](const lstk::LaunchTiming *tm) {
         return rows ? lstk::launch_gate_up_rows(gu, max_items, st, tm) : lstk::launch_gate_up_grouped(gu, max_items, st, tm);
     });

@@ -32,6 +32,9 @@ def _ids(rng, T, reps):
     ((12, 12, 12), 256, 256, 64), ((12, 12, 12), 4096, 256, 64), ((10, 10, 11), 256, 512, 64), ((11, 11, 10), 512, 256, 63),
     ((13, 13, 14), 512, 256, 64), ((14, 14, 13), 256, 256, 33), ((12, 12, 14), 2048, 768, 64), ((12, 12, 8), 512, 256, 64),
     ((8, 8, 14), 256, 256, 320), ((10, 10, 11), 4096, 256, 64),
+    # up to 4 pairs per expert the weights are read with the non-temporal hint; each format at its fewest tokens
+    ((8, 8, 8), 256, 256, 32), ((8, 8, 8), 4096, 256, 32), ((12, 12, 8), 512, 256, 32), ((12, 12, 12), 1024, 512, 9),
+    ((12, 12, 14), 1024, 512, 12), ((10, 10, 11), 1024, 512, 17), ((11, 11, 10), 4096, 256, 17),
 ], ids=lambda v: "-".join(map(str, v)) if isinstance(v, tuple) else str(v))
 def test_rows_ffn_matches_oracle(orc, lstk, dev, types, h, f, T):
     import torch
