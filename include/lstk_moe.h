@@ -203,7 +203,7 @@ int lstk_moe_block_noalloc(lstk_pool *pool, int layer, const float *d_hnorm, con
  * bin d_bins[t][j] in [0, n_bins), bins ascending and each bin's pairs in token-major order (a stable
  * counting sort). Writes d_counts [n_bins], d_offsets [n_bins + 1] (exclusive scan of the counts) and
  * d_perm [n_tokens * n_expert_used] (sorted position -> pair index). n_bins <= 1024. A bin out of range
- * is clamped on the device and reported by lstk_pool_check. The grouped (prefill) path of
+ * is clamped on the device and reported by lstk_pool_check. The grouped (many-token) path of
  * lstk_moe_ffn / lstk_moe_block runs the same kernel. */
 int lstk_moe_permute(lstk_pool *pool, const int32_t *d_bins, int n_tokens, int n_bins, int32_t *d_counts,
                      int32_t *d_offsets, int32_t *d_perm, lstk_stream_t stream);

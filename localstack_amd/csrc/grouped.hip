@@ -2,10 +2,11 @@
 // each expert. ggml's CPU mul_mat_id groups the (token, slot) pairs by expert and runs each expert's
 // matrix over its rows (src/qwen3.cpp:201-204); here that is:
 //   permute    one work-group: per-bin counts, exclusive offsets, the stable token-major pair order
-//              and the work list of 32-pair chunks, expert-major (each expert's chunks in order).
+//              and the work list of 16- or 32-pair chunks, expert-major (each expert's chunks in order).
+//   act_quant  the SwiGLU rows to Q8_K or Q8_0, the activation type ggml pairs with the down weights.
+// and, for Q4_K layers with many pairs per expert (the other calls' products: grouped_rows.hip),
 //   gate_up    per (chunk, 64-row block): Q4_K gate and up rows x Q8_K token rows on
 //              v_mfma_i32_32x32x32_i8, fused SwiGLU (src/qwen3.cpp:201-203).
-//   act_quant  the SwiGLU rows to Q8_K, the activation type ggml pairs with Q4_K down weights.
 //   down       per (chunk, 128-row block): Q4_K down rows x Q8_K SwiGLU rows, times the router
 //              weight (src/qwen3.cpp:204-205). The existing combine kernel sums the k rows.
 //

@@ -129,7 +129,8 @@ struct PermuteParams {
     int limit;        // > 0: a bin with more pairs sets bit 2 of *err (as the GEMV path's kernels do past T)
 };
 
-// One grouped expert product over the work list: Q4_K weight rows x Q8_K activation rows on MFMA.
+// One grouped expert product over the work list on MFMA: Q8_0 rows x Q8_0 activations, Q4_K or KQ8 rows x Q8_K
+// (the LDS-staged kernels of grouped.hip: Q4_K only).
 // gate_up: w0 = gate, w1 = up, activation row of a pair = its token (pair / k), out = SwiGLU rows
 // [np][rows]. down: w0 = down, activation row = the pair, out = weighted rows [np][rows].
 struct GroupedParams {
@@ -142,7 +143,7 @@ struct GroupedParams {
     int rows, K;             // weight matrix rows x K (= cols)
     const int8_t *xqs;       // activation rows [*][K] int8
     const float *xd;         // [*][K / 32], the Q8_K scale of each super-block repeated 8 times
-    const uint32_t *xbh;     // [*][K / 32], the 32-value group sums as split_sum_f16 pairs
+    const uint32_t *xbh;     // [*][K / 32], the 32-value group sums as split_sum_f16 pairs (Q8_K only)
     int row_div;             // activation row = pair / row_div
     const float *weights;    // down: router weight of each pair
     float *out;
@@ -239,14 +240,14 @@ int tier_copy_chunks(size_t bytes);
 hipError_t launch_tier_resolve(const TierResolveParams &p, hipStream_t s, const LaunchTiming *t);
 hipError_t launch_tier_copy(const TierCopyParams &p, hipStream_t s, const LaunchTiming *t);
 
-// grouped (prefill) path, grouped.hip
+// grouped (many-token) path: permute, act_quant and the LDS-staged Q4_K products, grouped.hip
 #ifndef LSTK_GROUPED_CHUNK
 #define LSTK_GROUPED_CHUNK 32
 #endif
-constexpr int kGroupedChunk = LSTK_GROUPED_CHUNK; // pairs per work item (32 or 64)
+constexpr int kGroupedChunk = LSTK_GROUPED_CHUNK; // pairs per work item of the staged kernels (32 or 64)
 constexpr int kGroupedMaxBins = 1024;    // bins the permutation kernel handles
-// True when the grouped MFMA kernels handle this layer: Q4_K gate, up and down, f % 64 == 0,
-// n_bins <= kGroupedMaxBins.
+// True when the grouped MFMA kernels handle this layer: gate and up of one pool format, any down format, h and f
+// multiples of 256, n_bins <= kGroupedMaxBins.
 bool grouped_supported(int tu, int tg, int td, int h, int f, int n_bins);
 // Upper bound on the work items of np pairs over n_bins bins.
 int grouped_max_items(int np, int n_bins, int chunk);

@@ -188,7 +188,7 @@ struct lstk_pool {
     uint8_t *noalloc = nullptr;
     int32_t *err = nullptr;
     int n_bins_max = 0;
-    // grouped (prefill) path: permutation, work list, Q8_K SwiGLU rows
+    // grouped (many-token) path: permutation, work list, quantized SwiGLU rows
     int32_t *counts = nullptr, *offsets = nullptr, *perm = nullptr, *n_items = nullptr;
     int4 *items = nullptr;
     lstk::ActBuf aq{};

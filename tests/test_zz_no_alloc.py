@@ -23,7 +23,7 @@ def _outs(torch, dev, T, h, k):
 
 @pytest.mark.parametrize("wtype,h,f,E,k,n_batch,calls", [
     (8, 2048, 768, 128, 8, 16, (8, 1)),     # 30B-A3B shape, Q8_0: batch then single token
-    (12, 2048, 768, 128, 8, 64, (48, 5)),  # Q4_K experts, batch sizes below the grouped threshold
+    (12, 2048, 768, 128, 8, 64, (48, 5)),  # Q4_K experts: the grouped path and the GEMV path
     (8, 256, 512, 8, 2, 16, (16, 3)),       # tiny qwen3moe shape
 ])
 def test_noalloc_block_matches_block(lstk, dev, wtype, h, f, E, k, n_batch, calls):
