@@ -1035,7 +1035,7 @@ int run_grouped(lstk_pool *P, const Shard &s, const CallScratch &sc, bool fixed,
         return rows ? lstk::launch_down_rows(dn, max_items, st, tm) : lstk::launch_down_grouped(dn, max_items, st, tm);
     });
     if (e != hipSuccess) return hip_fail(e, "down launch");
-    if (P->defer_combine && !fixed) return LSTK_OK;
+    if (P->defer_combine && !fixed && T > 1) return LSTK_OK;
     lstk::CombineParams cp{sc.Y, d_resid, d_out, T, k, h};
     e = timed(P, 3, [&](const lstk::LaunchTiming *tm) { return lstk::launch_combine(cp, st, tm); });
     if (e != hipSuccess) return hip_fail(e, "combine launch");
@@ -1078,7 +1078,7 @@ int run_block(lstk_pool *P, int layer, int mode, const float *d_hnorm, const voi
     rp.xq.bh = grouped ? P->xq.bh : nullptr; // only the grouped kernels read the split group sums
     hipError_t e = timed(P, 0, [&](const lstk::LaunchTiming *tm) { return lstk::launch_route(rp, st, tm); });
     if (e != hipSuccess) return hip_fail(e, "route launch");
-    const bool fused_topk = mode == 1 && T <= lstk::decode_route_max_tokens();
+    const bool fused_topk = mode == 1 && !grouped && T <= lstk::decode_route_max_tokens(); // grouped reads d_ids
     if (mode == 1 && !fused_topk) {
         lstk::TopkParams tp{sc.logits, T, d.n_expert, k, d_ids, d_weights};
         e = timed(P, 0, [&](const lstk::LaunchTiming *tm) { return lstk::launch_topk(tp, st, tm); });

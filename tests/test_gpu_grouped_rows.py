@@ -59,3 +59,29 @@ def test_rows_ffn_matches_oracle(orc, lstk, dev, types, h, f, T):
     err = np.abs(outs[0] - ref).max() / np.abs(ref - resid).max()
     print(f"[rows {types} h={h} f={f} T={T}] rel max err {err:.3e}", flush=True)
     assert err <= FFN_TOL * max(1.0, (512 / f) ** 0.5)
+
+
+@pytest.mark.parametrize("wtype", (8, 12))
+def test_one_token_block_with_the_threshold_at_one(lstk, dev, monkeypatch, wtype):
+    """LSTK_GROUPED_MIN_TOKENS=1: a one-token block on the matrix cores routes before it groups (same ids and weights as
+    the default path, outputs to the f32 order over super-blocks)."""
+    import torch
+    h, f, E, k = 256, 512, 16, 2
+    rng = np.random.default_rng(7 + wtype)
+    mats = [synth.experts(rng, wtype, E, r, c, centered=True) for r, c in ((f, h), (f, h), (h, f))]
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    x, resid = d(synth.activations(rng, 1, h)), d(synth.activations(rng, 1, h))
+    gate = d(rng.normal(0, 0.05, (E, h)).astype(np.float32))
+    got = []
+    for env in (None, "1"):
+        if env:
+            monkeypatch.setenv("LSTK_GROUPED_MIN_TOKENS", env)
+        store = lstk.ExpertStore(1, h, f, E, k, 1, [((wtype,) * 3, *mats)])
+        out = torch.full((1, h), np.nan, dtype=torch.float32, device=dev)
+        ids, w = torch.full((1, k), -7, dtype=torch.int32, device=dev), torch.zeros(1, k, device=dev)
+        store.block(0, x, gate, lstk.TYPE_F32, resid, out, ids, w)
+        store.check()
+        got.append([t.cpu().numpy() for t in (out, ids, w)])
+        store.close()
+    assert np.array_equal(got[0][1], got[1][1]) and np.array_equal(got[0][2], got[1][2])
+    assert np.abs(got[0][0] - got[1][0]).max() <= FFN_TOL * np.abs(got[0][0] - resid.cpu().numpy()).max()
