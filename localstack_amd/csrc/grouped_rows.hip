@@ -13,7 +13,9 @@
 //   Q8_0  acc += d_x (d_w I). The product starts from the constant accumulator 0x4b400000, the bits of 1.5 2^23: its
 //         int32 result read as a float is 1.5 2^23 + I exactly (|I| <= 516128), so one fma with the exact addend
 //         -1.5 2^23 d_w gives d_w I rounded once, and a second one adds d_x of it: two VALU operations per output
-//         and block instead of convert, multiply and fma.
+//         and block instead of convert, multiply and fma. A super-block's eight blocks are summed on their own and
+//         the super-blocks after that, as the GEMV kernels' threads do: one chain over the 64 blocks of K 2048 would
+//         round 1.7 times as far from 64 bits (1.45e-7 of the result against 0.83e-7, and 0.80e-7 as it is).
 //   Q4_K  isum += sc I (24-bit multiply-add, exact), imin on one v_mfma_f32_16x16x32_f16 per super-block over the split
 //         group sums (exact integers, as in grouped.hip), then acc += d_x (d_w isum - dmin imin).
 //   KQ8   scales per 16 values: two products per block, each seeing the tokens of one half of K and zeros for the
@@ -161,13 +163,11 @@ __device__ __forceinline__ void stage_rows(const GroupedParams &P, const RLds &L
     }
 }
 
-// The activations of block b (0 .. 7) of a super-block for the lane: 8 bytes of row r of every M-tile and, for Q8_0, the
-// block's scales of rows 4 kg .. 4 kg + 3. KQ8 takes the two 16-value groups apart: lanes kg < 2 hold the first
+// The activations of block b (0 .. 7) of a super-block for the lane: 8 bytes of row r of every M-tile. KQ8 takes the two 16-value groups apart: lanes kg < 2 hold the first
 // (the others zeros), lanes kg >= 2 the second.
 template <int WT, int MT>
 struct Acts {
     uint2 a[WT == kTypeKQ8 ? 2 : 1][MT];
-    f32x4 dx[WT == kTypeQ8_0 ? MT : 0];
 };
 template <int WT, int MT, int CH>
 __device__ __forceinline__ void load_acts(Acts<WT, MT> &x, const RLds &L, int K, int sb, int b) {
@@ -183,7 +183,6 @@ __device__ __forceinline__ void load_acts(Acts<WT, MT> &x, const RLds &L, int K,
         } else {
             x.a[0][mt] = *reinterpret_cast<const uint2 *>(L.a + (at ^ (b * 32)));
         }
-        if constexpr (WT == kTypeQ8_0) x.dx[mt] = *reinterpret_cast<const f32x4 *>(L.dx + (sb * 8 + b) * CH + 16 * mt + 4 * kg);
     }
 }
 
@@ -227,13 +226,14 @@ __device__ __forceinline__ void rows_products(const RLds &L, int K, const uint8_
     load_acts<WT, MT, CH>(x, L, K, 0, 0);
     auto super_block = [&](int sb, auto more_c) __attribute__((always_inline)) {
         constexpr bool more = decltype(more_c)::value;
-        TileH<WT, MINS> nh[2];
+        TileH<WT, MINS> nh[2]; // (not Q8_0)
 #pragma unroll
         for (int t = 0; t < 2; t++) {
             wp[t] += C * 256;
-            if constexpr (more) load_h<WT, MINS, NT>(nh[t], wp[t]);
+            if constexpr (more && WT != kTypeQ8_0) load_h<WT, MINS, NT>(nh[t], wp[t]);
         }
         i32x4 isum[2][WT == kTypeQ8_0 ? 0 : MT], imin[2][WT == kTypeKQ8 && MINS ? MT : 0];
+        f32x4 part[2][WT == kTypeQ8_0 ? MT : 0]; // the super-block's own sum
         unsigned sc[2][2]; // Q4_K: the 6-bit scales, one per byte (sub-blocks 0-3 and 4-7)
         if constexpr (WT != kTypeQ8_0) {
 #pragma unroll
@@ -255,6 +255,9 @@ __device__ __forceinline__ void rows_products(const RLds &L, int K, const uint8_
             if constexpr (WT == kTypeQ8_0) {
                 float d[2], c[2];
                 i32x4 I[2][MT];
+                f32x4 dx[MT]; // arrive during the products
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++) dx[mt] = *reinterpret_cast<const f32x4 *>(L.dx + (sb * 8 + b) * CH + 16 * mt + 4 * kg);
 #pragma unroll
                 for (int t = 0; t < 2; t++) {
                     const unsigned d2 = here(dw(h[t].h, b / 2));
@@ -268,12 +271,14 @@ __device__ __forceinline__ void rows_products(const RLds &L, int K, const uint8_
 #pragma unroll
                     for (int t = 0; t < 2; t++)
 #pragma unroll
-                        for (int i = 0; i < 4; i++)
-                            acc[t][mt][i] = fmaf(x.dx[mt][i], fmaf(__int_as_float(I[t][mt][i]), d[t], c[t]), acc[t][mt][i]);
+                        for (int i = 0; i < 4; i++) {
+                            const float v = fmaf(__int_as_float(I[t][mt][i]), d[t], c[t]);
+                            part[t][mt][i] = b == 0 ? dx[mt][i] * v : fmaf(dx[mt][i], v, part[t][mt][i]);
+                        }
 #pragma unroll
                 for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-                    for (int t = 0; t < 2; t++) pin(acc[t][mt]);
+                    for (int t = 0; t < 2; t++) pin(part[t][mt]);
             } else if constexpr (WT == kTypeQ4_K) {
                 i32x4 I[2][MT];
                 int s[2];
@@ -334,12 +339,26 @@ __device__ __forceinline__ void rows_products(const RLds &L, int K, const uint8_
                         q[t].q[bq] = load_q<WT, NT>(wp[t], bq);
                     }
                 }
+                // Q8_0: the scales of blocks 0-3 and 4-7 likewise, as soon as their last block is done
+                if (WT == kTypeQ8_0 && b % 4 == 3) {
+#pragma unroll
+                    for (int t = 0; t < 2; t++) {
+                        const uint2 v = load_w<NT, uint2>(wp[t] + r * 16 + 2 * (b - 3));
+                        if (b == 3) h[t].h.x = v.x, h[t].h.y = v.y;
+                        else h[t].h.z = v.x, h[t].h.w = v.y;
+                    }
+                }
             }
             if (b < 7 || more) x = nx;
             asm volatile("" ::: "memory"); // the next block's reads stay behind this one's products
             __builtin_amdgcn_sched_barrier(0);
         }
-        if constexpr (WT == kTypeQ4_K) {
+        if constexpr (WT == kTypeQ8_0) {
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++) acc[t][mt] += part[t][mt];
+        } else if constexpr (WT == kTypeQ4_K) {
             f32x4 fmin[2][MT];
 #pragma unroll
             for (int t = 0; t < 2; t++) {
@@ -385,7 +404,7 @@ __device__ __forceinline__ void rows_products(const RLds &L, int K, const uint8_
                 }
             }
         }
-        if constexpr (more) {
+        if constexpr (more && WT != kTypeQ8_0) {
             h[0] = nh[0];
             h[1] = nh[1];
         }

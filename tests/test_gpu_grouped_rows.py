@@ -85,3 +85,47 @@ def test_one_token_block_with_the_threshold_at_one(lstk, dev, monkeypatch, wtype
         store.close()
     assert np.array_equal(got[0][1], got[1][1]) and np.array_equal(got[0][2], got[1][2])
     assert np.abs(got[0][0] - got[1][0]).max() <= FFN_TOL * np.abs(got[0][0] - resid.cpu().numpy()).max()
+
+
+@pytest.mark.parametrize("E", (2, 16), ids=("32-pair items", "16-pair items"))
+def test_q8_0_sums_are_as_close_to_64_bits_as_the_gemv_paths(lstk, dev, E):
+    """The f32 rounding of a Q8_0 row's sum over K 2048 (64 blocks), against 64 bits, is no larger than the GEMV path's
+    (each expert's first 8 tokens of a call of 8). Token t is column t of the activations, gate is constant and up holds
+    integers with 127 in every 32-row block, so the SwiGLU row quantizes to up's column t exactly and every block has the
+    same scale: what the outputs differ by is the down product's own rounding. 5% for the two estimates of 64 x 256 values."""
+    import torch
+    h, f, k, T = 256, 2048, 1, 64
+    rng = np.random.default_rng(5 + E)
+
+    def blocks(q, d):  # q [rows, cols] integers, d [rows, cols / 32] -> GGUF Q8_0 bytes
+        out = np.empty(q.shape[:1] + (q.shape[1] // 32, 34), np.uint8)
+        out[..., :2] = d.astype(np.float16)[..., None].view(np.uint8)
+        out[..., 2:] = q.astype(np.int8).reshape(out.shape[:2] + (32,)).view(np.uint8)
+        return out.reshape(-1)
+
+    up_q = rng.integers(-127, 128, (f, h))
+    up_q[::32] = 127
+    down_q = np.clip(np.rint(rng.normal(0, 45, (h, f))), -127, 127).astype(np.int64)
+    down_d = (0.02 * rng.uniform(0.8, 1.2, (h, f // 32)) / 45).astype(np.float16)
+    gate = np.tile(blocks(np.full((f, h), 100), np.full((f, h // 32), 0.02)), E)
+    up, down = np.tile(blocks(up_q, np.full((f, h // 32), 0.01)), E), np.tile(blocks(down_q, down_d), E)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    x = np.eye(T, h, dtype=np.float32)
+    # sum over blocks of d_w I in 64 bits; the rows' common scale is one fp16 value
+    ref = np.einsum("tbi,rbi,rb->tr", up_q[:, :T].T.reshape(T, -1, 32), down_q.reshape(h, -1, 32), down_d.astype(np.float64), optimize=True)
+    store = lstk.ExpertStore(1, h, f, E, k, T, [((8, 8, 8), up, gate, down)])
+    err = []
+    for step in (T, 8):
+        out = np.empty((T, h))
+        for t in range(0, T, step):
+            o = torch.full((step, h), np.nan, device=dev)
+            store.ffn(0, d(x[t:t + step]), torch.zeros(step, k, dtype=torch.int32, device=dev), torch.ones(step, k, device=dev),
+                      torch.zeros(step, h, device=dev), o)
+            store.check()
+            out[t:t + step] = o.cpu().numpy()
+        s = float(np.float16((out * ref).sum() / (ref * ref).sum()))
+        err.append(np.sqrt(np.mean((out - s * ref) ** 2) / np.mean((s * ref) ** 2)))
+    store.close()
+    print(f"[Q8_0 K={f} E={E}] error against 64 bits: many tokens {err[0]:.3e}, GEMV {err[1]:.3e}", flush=True)
+    assert err[1] < 2e-7, "the quantized rows are not the integers this test assumes"
+    assert err[0] <= 1.05 * err[1]
