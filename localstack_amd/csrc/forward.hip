@@ -1204,8 +1204,9 @@ __global__ __launch_bounds__(kAtBlock) void attn_rows_kernel(AttnParams P) {
 //
 // A 32-cell block is live for the work-group when some cell of it belongs to the sequence at a position its last row
 // sees: other sequences' blocks and those above the causal diagonal cost nothing. The live blocks are taken in the
-// order of their positions (a block holds consecutive positions of one sequence from its first cell), so a chunk's sums
-// do not depend on the order its blocks lie in. Where a unit is seen whole (every
+// order of their positions (a block holds positions 32 i .. 32 i + 31 of one sequence, position p in its cell p % 32), so
+// the sums of a chunk do not depend on the order its blocks lie in. (Chunks are cut by cell: which blocks meet in one does
+// depend on it, where a launch has more than one chunk per row block.) Where a unit is seen whole (every
 // cell the sequence's, none past the row block's first row) its scores skip the visibility tests.
 //
 // The softmax runs in base 2 against a running maximum raised to the next integer: p = 2^(s c - m) with c = scale log2 e
@@ -1295,9 +1296,12 @@ __global__ __launch_bounds__(kAsWaves *kWave) void attn_split_kernel(AttnParams 
                 const int pass = p0 + u * kAsWaves + wave;
                 const unsigned long long mk =
                     __ballot(pass < n_pass && cs[u] == P.seq && cp[u] <= pos_last && begin + pass * kFaCells + l < end);
-                const int blk = 2 * pass + (l >> 5), key = by_pos ? cp[u] / 32 : blk;
-                // (lanes 0 and 32: their cells are the blocks' first, with the lowest positions)
-                if ((l & 31) == 0 && (unsigned) (mk >> (l & 32)) != 0u && key >= 0 && key < n_at) S.at[key] = (uint16_t) blk;
+                // lanes 0 and 32 write their blocks' entries. The position is that of the block's first live cell: its first
+                // cells may hold none (reserved by a step that has not run)
+                const unsigned live = (unsigned) (mk >> (l & 32));
+                const int first = __shfl(cp[u], (l & 32) + max(__ffs((int) live) - 1, 0), kWave);
+                const int blk = 2 * pass + (l >> 5), key = by_pos ? first / 32 : blk;
+                if ((l & 31) == 0 && live != 0u && key >= 0 && key < n_at) S.at[key] = (uint16_t) blk;
             }
         }
         __syncthreads();

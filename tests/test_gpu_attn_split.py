@@ -34,3 +34,23 @@ def test_prompt_steps_match_oracle(lstk, dev, steps, shared):
         model.truncate_seq(7, 33)
     for i, n in enumerate(steps):
         _check(ref, model, 0, prompt(100 * i + n, n, hp["n_vocab"]), hp, dev, f"shared {shared} step {i} of {n}")
+
+
+def test_block_whose_first_cells_were_never_written(lstk, dev):
+    """32 tokens, then 5 cells reserved by a prepare whose forward never ran, then a 91-token step: the second block's first
+    cells hold no position, and the step sees its other cells and the first block as steps of 30 tokens do (attn_rows_kernel;
+    f32 orders apart, so the bar is the forward pass's own)."""
+    hp, w = weights("tiny")
+    toks, lg = prompt(3, 32 + 91, hp["n_vocab"]), []
+    for steps in ((91,), (30, 30, 31)):
+        _, model = build(lstk, dev, hp, w, n_batch=96, kv_size=512)
+        run(model, 0, toks[:32], hp, dev)
+        model.prepare(0, toks[:5])
+        at = 32
+        for n in steps:
+            out, _ = run(model, 0, toks[at:at + n], hp, dev)
+            at += n
+        lg.append(out)
+    err, rms, ra, ga = oracle.diff_logits(*lg)
+    print(f"[hole] max|dlogit| {err:.2e} rms {rms:.2e} top1 {ga}/{ra}", flush=True)
+    assert err <= LOGITS_TOL and rms <= RMS_TOL and ga == ra
