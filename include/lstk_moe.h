@@ -183,11 +183,11 @@ int lstk_moe_block(lstk_pool *pool, int layer, const float *d_hnorm, const void 
 
 /* No counterpart in the reference: lstk_moe_block for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). The call's
- * scratch (quantized activations, router logits, SwiGLU rows, per-pair outputs) comes from a fixed
- * array of LSTK_NOALLOC_SCRATCH_BYTES in the library, one copy per device, held until the process
- * ends (a call of many tokens also uses the pool's own work list and quantized SwiGLU rows, laid out at
- * creation); the call allocates nothing and creates no events. Same arguments, kernels and results as
- * lstk_moe_block, except that it never takes the fused path and keeps no stage timing. Fails with
+ * scratch (quantized activations, router logits, SwiGLU rows, per-pair outputs, a many-token call's work list) comes
+ * from a fixed array of LSTK_NOALLOC_SCRATCH_BYTES in the library, one copy per device, held until the process ends;
+ * the call allocates nothing and creates no events. Same arguments, kernels and results as lstk_moe_block, except
+ * that it never takes the fused path, keeps no stage timing, and takes the grouped path only where the array holds that
+ * path's work list, quantized SwiGLU rows and group sums too (at the 30B-A3B shape up to 164 tokens). Fails with
  * LSTK_E_INVALID when n_tokens needs more scratch than the array holds:
  * n_tokens * (n_embd * (1.25 + 4 k) + 4 E + 4 k n_ff_exp) bytes, each part rounded up to 256
  * (up to 180 tokens at the 30B-A3B shape, 90 at the 235B-A22B shape; n_batch of the pool still
@@ -239,6 +239,12 @@ int lstk_unpack_matrix(int type, int rows, int cols, const void *packed, void *g
  * src/expert_store.cpp:62-66): the next n host-tier copies fail, the acquire returns LSTK_E_IO and
  * the slots involved are unmapped. */
 int lstk_pool_debug_fail_copies(lstk_pool *pool, int n);
+
+/* Test hook (no counterpart in the reference): how an expert call of n_tokens runs on a shard of n_slots slots with these
+ * types (host arithmetic only, no device call; dims->n_layer and n_batch are not read). out[0..4] = grouped path (0 / 1),
+ * its products on the register-streaming kernels (0: the LDS-staged ones), pairs per work item, weights with the
+ * non-temporal hint, grouped in lstk_moe_block_noalloc too. */
+int lstk_debug_moe_plan(const lstk_moe_dims *dims, int type_gate, int type_down, int n_slots, int n_tokens, int32_t out[5]);
 
 #ifdef __cplusplus
 }

@@ -131,6 +131,7 @@ SIGNATURES = {
     "lstk_dequant_f16": (_I, [_I, _P, ctypes.c_size_t, _P]),
     "lstk_model_set_timing": (_I, [_P, _I]),
     "lstk_debug_attn_plan": (_I, [_I, _I, _I, _I, _I, _I, _I, _I, _P]),
+    "lstk_debug_moe_plan": (_I, [ctypes.POINTER(MoeDims), _I, _I, _I, _I, _P]),
     "lstk_model_debug_options": (_I, [_P, _I]),
     "lstk_model_timing": (_I, [_P, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_int64)]),
 }
@@ -211,6 +212,16 @@ def attn_plan(n_tokens, n_head, n_kv, head_dim, kv_size, n_cells, cell_begin=0, 
     _check(lib().lstk_debug_attn_plan(int(n_tokens), int(n_head), int(n_kv), int(head_dim), int(kv_size), int(n_cells),
                                       int(cell_begin), 1 if rope_in else 0, ctypes.cast(out, ctypes.c_void_p)))
     return out[0], out[1], out[2], out[3], bool(out[4]), out[5]
+
+
+def moe_plan(types, n_embd, n_ff_exp, n_expert, n_expert_used, n_tokens, n_slots=None):
+    """How an expert call of n_tokens runs (host arithmetic, no device call): (grouped path, register-streaming kernels,
+    pairs per work item, non-temporal weights, grouped in block_noalloc too). types = (up, gate, down)."""
+    d = MoeDims(1, int(n_embd), int(n_ff_exp), int(n_expert), int(n_expert_used), int(n_tokens))
+    out = (ctypes.c_int32 * 5)()
+    _check(lib().lstk_debug_moe_plan(ctypes.byref(d), int(types[1]), int(types[2]), int(n_slots or n_expert), int(n_tokens),
+                                     ctypes.cast(out, ctypes.c_void_p)))
+    return bool(out[0]), bool(out[1]), out[2], bool(out[3]), bool(out[4])
 
 
 def repack_matrix(type_, rows, cols, gguf):

@@ -153,6 +153,15 @@ constexpr int kSides = LSTK_SIDE_STREAMS;
 constexpr size_t kNoAllocBytes = LSTK_NOALLOC_SCRATCH_BYTES;
 static __device__ __align__(256) uint8_t scratch[kNoAllocBytes];
 
+// What the grouped (many-token) path needs beside the GEMV path's scratch: permutation, work list, quantized SwiGLU rows,
+// split group sums of the activations.
+struct GroupedScratch {
+    int32_t *counts, *offsets, *perm, *n_items;
+    int4 *items;
+    lstk::ActBuf aq;
+    uint32_t *xbh;
+};
+
 struct lstk_pool {
     lstk_moe_dims dims{};
     bool streaming = false, dry = false;
@@ -188,10 +197,7 @@ struct lstk_pool {
     uint8_t *noalloc = nullptr;
     int32_t *err = nullptr;
     int n_bins_max = 0;
-    // grouped (many-token) path: permutation, work list, quantized SwiGLU rows
-    int32_t *counts = nullptr, *offsets = nullptr, *perm = nullptr, *n_items = nullptr;
-    int4 *items = nullptr;
-    lstk::ActBuf aq{};
+    GroupedScratch grouped{};
     int grouped_min_tokens = 0;
     // fused single-token path: launch counters and stage flags (zero at creation)
     lstk::FusedLayout fl{};
@@ -209,6 +215,35 @@ namespace {
 
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
+// Bytes of a GroupedScratch for T tokens over n_bins bins, and its layout from `base` when base is non-null.
+size_t grouped_scratch(const lstk_moe_dims &d, int T, int n_bins, uint8_t *base, GroupedScratch *out) {
+    const size_t t = (size_t) T, np = t * (size_t) d.n_expert_used, nb = (size_t) n_bins;
+    const size_t h = (size_t) d.n_embd, f = (size_t) d.n_ff_exp;
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        const size_t o = off;
+        off = align_up(off + bytes, 256);
+        return base + o;
+    };
+    uint8_t *counts = take(nb * 4), *offsets = take((nb + 1) * 4), *perm = take(np * 4), *n_items = take(64);
+    uint8_t *items = take((size_t) lstk::grouped_max_items((int) np, n_bins, 16) * 16); // 16: the shortest work items
+    uint8_t *qs = take(np * f), *ad = take(np * (f / 32) * 4), *bs = take(np * (f / 32) * 4), *bh = take(np * (f / 32) * 4);
+    uint8_t *xbh = take(t * (h / 32) * 4);
+    if (base && out) {
+        out->counts = reinterpret_cast<int32_t *>(counts);
+        out->offsets = reinterpret_cast<int32_t *>(offsets);
+        out->perm = reinterpret_cast<int32_t *>(perm);
+        out->n_items = reinterpret_cast<int32_t *>(n_items);
+        out->items = reinterpret_cast<int4 *>(items);
+        out->aq.qs = reinterpret_cast<int8_t *>(qs);
+        out->aq.d = reinterpret_cast<float *>(ad);
+        out->aq.bs = reinterpret_cast<int32_t *>(bs);
+        out->aq.bh = reinterpret_cast<uint32_t *>(bh);
+        out->xbh = reinterpret_cast<uint32_t *>(xbh);
+    }
+    return off;
+}
+
 int alloc_scratch(lstk_pool *P) {
     const lstk_moe_dims &d = P->dims;
     const size_t nb = (size_t) P->n_bins_max, T = (size_t) d.n_batch, k = (size_t) d.n_expert_used;
@@ -220,16 +255,10 @@ int alloc_scratch(lstk_pool *P) {
         return o;
     };
     const size_t o_qs = take(T * h), o_d = take(T * (h / 32) * 4), o_bs = take(T * (h / 32) * 4);
-    const size_t o_bh = take(T * (h / 32) * 4);
     const size_t o_logits = take(T * E * 4);
     const size_t o_act = take(T * k * f * 4), o_Y = take(T * k * h * 4);
     const size_t o_err = take(64);
-    const size_t np = T * k;
-    const size_t max_items = (size_t) lstk::grouped_max_items((int) np, (int) nb, 16);
-    const size_t o_counts = take(nb * 4), o_offsets = take((nb + 1) * 4), o_perm = take(np * 4), o_nitems = take(64);
-    const size_t o_items = take(max_items * 16);
-    const size_t o_aqs = take(np * f), o_ad = take(np * (f / 32) * 4), o_abs = take(np * (f / 32) * 4);
-    const size_t o_abh = take(np * (f / 32) * 4);
+    const size_t o_grouped = take(grouped_scratch(d, d.n_batch, (int) nb, nullptr, nullptr));
     P->fl = lstk::fused_layout((int) h, (int) f, (int) E, (int) k);
     const size_t n_fused = P->fl.ok ? (size_t) (P->fl.nB + P->fl.nC) : 1;
     const size_t o_fcnt = take(n_fused * 4), o_fa = take((size_t) std::max(P->fl.nA, 1) * 4),
@@ -242,20 +271,11 @@ int alloc_scratch(lstk_pool *P) {
     P->xq.qs = reinterpret_cast<int8_t *>(b + o_qs);
     P->xq.d = reinterpret_cast<float *>(b + o_d);
     P->xq.bs = reinterpret_cast<int32_t *>(b + o_bs);
-    P->xq.bh = reinterpret_cast<uint32_t *>(b + o_bh);
     P->logits = reinterpret_cast<float *>(b + o_logits);
     P->act = reinterpret_cast<float *>(b + o_act);
     P->Y = reinterpret_cast<float *>(b + o_Y);
     P->err = reinterpret_cast<int32_t *>(b + o_err);
-    P->counts = reinterpret_cast<int32_t *>(b + o_counts);
-    P->offsets = reinterpret_cast<int32_t *>(b + o_offsets);
-    P->perm = reinterpret_cast<int32_t *>(b + o_perm);
-    P->n_items = reinterpret_cast<int32_t *>(b + o_nitems);
-    P->items = reinterpret_cast<int4 *>(b + o_items);
-    P->aq.qs = reinterpret_cast<int8_t *>(b + o_aqs);
-    P->aq.d = reinterpret_cast<float *>(b + o_ad);
-    P->aq.bs = reinterpret_cast<int32_t *>(b + o_abs);
-    P->aq.bh = reinterpret_cast<uint32_t *>(b + o_abh);
+    grouped_scratch(d, d.n_batch, (int) nb, b + o_grouped, &P->grouped);
     P->f_cnt = reinterpret_cast<int *>(b + o_fcnt);
     P->f_flag_a = reinterpret_cast<int *>(b + o_fa);
     P->f_flag_b = reinterpret_cast<int *>(b + o_fb);
@@ -843,18 +863,23 @@ int check_call(lstk_pool *P, int layer, int T) {
 //   Q8_0: 24 101 / 112 and 86 / 61, 32 118 / 126 and 114 / 59, 48 147 / 140.
 // Experts below a million weights (the tiny shapes) are cheap either way, so their calls keep the fewer launches up to
 // 31 tokens (h 256, f 512, 8 experts, Q8_0: 17 tokens 28 / 35, 32 40 / 34).
-int grouped_from(const Shard &s, int h, int f) {
-    if ((long) 3 * h * f < 1000000 || s.tg == lstk::kTypeQ8_0) return 32;
-    if (s.tg != lstk::kTypeQ4_K) return 17;
-    return s.td == lstk::kTypeQ4_K ? 9 : s.td == lstk::kTypeQ8_0 ? 32 : 12;
+int grouped_from(int tg, int td, int h, int f) {
+    if ((long) 3 * h * f < 1000000 || tg == lstk::kTypeQ8_0) return 32;
+    if (tg != lstk::kTypeQ4_K) return 17;
+    return td == lstk::kTypeQ4_K ? 9 : td == lstk::kTypeQ8_0 ? 32 : 12;
+}
+// LSTK_GROUPED_MIN_TOKENS, or -1 where it is not set.
+int grouped_env() {
+    const char *env = std::getenv("LSTK_GROUPED_MIN_TOKENS");
+    return env ? std::max(1, std::atoi(env)) : -1;
+}
+bool takes_grouped(const lstk_moe_dims &d, int tu, int tg, int td, int n_slots, int T, int env) {
+    return T >= (env > 0 ? env : grouped_from(tg, td, d.n_embd, d.n_ff_exp)) &&
+           lstk::grouped_supported(tu, tg, td, d.n_embd, d.n_ff_exp, n_slots);
 }
 bool use_grouped(lstk_pool *P, const Shard &s, int T) {
-    if (P->grouped_min_tokens == 0) {
-        const char *env = std::getenv("LSTK_GROUPED_MIN_TOKENS");
-        P->grouped_min_tokens = env ? std::max(1, std::atoi(env)) : -1;
-    }
-    const int from = P->grouped_min_tokens > 0 ? P->grouped_min_tokens : grouped_from(s, P->dims.n_embd, P->dims.n_ff_exp);
-    return T >= from && lstk::grouped_supported(s.tu, s.tg, s.td, P->dims.n_embd, P->dims.n_ff_exp, (int) s.n_slots);
+    if (P->grouped_min_tokens == 0) P->grouped_min_tokens = grouped_env();
+    return takes_grouped(P->dims, s.tu, s.tg, s.td, (int) s.n_slots, T, P->grouped_min_tokens);
 }
 
 // Which kernels run a many-token call's expert products, and the pairs per work item.
@@ -873,9 +898,9 @@ struct GroupedPlan {
     int chunk;
     bool once;
 };
-GroupedPlan grouped_plan(const Shard &s, int np, int n_expert) {
-    if (s.tg == lstk::kTypeQ4_K && s.td == lstk::kTypeQ4_K && np > 14 * n_expert) return {false, lstk::kGroupedChunk, false};
-    const bool q8 = s.tg == lstk::kTypeQ8_0 && s.td == lstk::kTypeQ8_0;
+GroupedPlan grouped_plan(int tg, int td, int np, int n_expert) {
+    if (tg == lstk::kTypeQ4_K && td == lstk::kTypeQ4_K && np > 14 * n_expert) return {false, lstk::kGroupedChunk, false};
+    const bool q8 = tg == lstk::kTypeQ8_0 && td == lstk::kTypeQ8_0;
     return {true, q8 && np > 12 * n_expert ? 32 : 16, np <= 4 * n_expert};
 }
 
@@ -951,9 +976,10 @@ struct NormIn {
 struct CallScratch {
     lstk::ActBuf xq;
     float *logits, *act, *Y;
+    GroupedScratch grouped; // counts null: the call does not take the grouped path
 };
 
-// Bytes of a CallScratch for T tokens, and its layout from `base` when base is non-null.
+// Bytes of a CallScratch for T tokens without its grouped part, and its layout from `base` when base is non-null.
 size_t call_scratch_layout(const lstk_moe_dims &d, int T, uint8_t *base, CallScratch *out) {
     const size_t t = (size_t) T, h = (size_t) d.n_embd, k = (size_t) d.n_expert_used;
     size_t off = 0;
@@ -976,9 +1002,14 @@ size_t call_scratch_layout(const lstk_moe_dims &d, int T, uint8_t *base, CallScr
     return off;
 }
 
+// Whether the fixed array holds the grouped part of a call of T tokens behind the rest.
+bool noalloc_grouped(const lstk_moe_dims &d, int n_bins, int T) {
+    return call_scratch_layout(d, T, nullptr, nullptr) + grouped_scratch(d, T, n_bins, nullptr, nullptr) <= kNoAllocBytes;
+}
+
 // permute -> gate_up (MFMA, SwiGLU) -> Q8_0 / Q8_K of the SwiGLU rows -> down (MFMA, router weight) ->
 // combine + residual. bins: expert ids (resident) or slots (streaming), [T][k].
-// fixed: the activations, SwiGLU rows and outputs are in the fixed array of lstk_moe_block_noalloc, no stage timing.
+// fixed: the scratch is in the fixed array of lstk_moe_block_noalloc, no stage timing.
 int run_grouped(lstk_pool *P, const Shard &s, const CallScratch &sc, bool fixed, const int32_t *bins, const float *d_weights,
                 const float *d_resid, float *d_out, int T, hipStream_t st) {
     auto timed = [&](lstk_pool *pool, int stage, auto &&launch) -> hipError_t {
@@ -986,16 +1017,17 @@ int run_grouped(lstk_pool *P, const Shard &s, const CallScratch &sc, bool fixed,
     };
     const lstk_moe_dims &d = P->dims;
     const int k = d.n_expert_used, np = T * k, h = d.n_embd, f = d.n_ff_exp;
-    const auto [rows, chunk, once] = grouped_plan(s, np, d.n_expert);
+    const auto [rows, chunk, once] = grouped_plan(s.tg, s.td, np, d.n_expert);
     const int max_items = lstk::grouped_max_items(np, (int) s.n_slots, chunk);
-    lstk::PermuteParams pp{bins, np, (int) s.n_slots, chunk, P->counts, P->offsets, P->perm,
-                           P->items, P->n_items, P->err, T < 64 || s.tg != lstk::kTypeQ4_K || s.td != lstk::kTypeQ4_K ? T : 0};
+    const GroupedScratch &g = sc.grouped;
+    lstk::PermuteParams pp{bins, np, (int) s.n_slots, chunk, g.counts, g.offsets, g.perm,
+                           g.items, g.n_items, P->err, T < 64 || s.tg != lstk::kTypeQ4_K || s.td != lstk::kTypeQ4_K ? T : 0};
     hipError_t e = timed(P, 0, [&](const lstk::LaunchTiming *tm) { return lstk::launch_permute(pp, st, tm); });
     if (e != hipSuccess) return hip_fail(e, "permute launch");
     lstk::GroupedParams gu{};
-    gu.items = P->items;
-    gu.n_items = P->n_items;
-    gu.perm = P->perm;
+    gu.items = g.items;
+    gu.n_items = g.n_items;
+    gu.perm = g.perm;
     gu.k = k;
     gu.w0 = s.d_gate;
     gu.w1 = s.d_up;
@@ -1005,7 +1037,7 @@ int run_grouped(lstk_pool *P, const Shard &s, const CallScratch &sc, bool fixed,
     gu.K = h;
     gu.xqs = sc.xq.qs;
     gu.xd = sc.xq.d;
-    gu.xbh = P->xq.bh;
+    gu.xbh = g.xbh;
     gu.row_div = k;
     gu.out = sc.act;
     gu.type = s.tg;
@@ -1015,7 +1047,7 @@ int run_grouped(lstk_pool *P, const Shard &s, const CallScratch &sc, bool fixed,
         return rows ? lstk::launch_gate_up_rows(gu, max_items, st, tm) : lstk::launch_gate_up_grouped(gu, max_items, st, tm);
     });
     if (e != hipSuccess) return hip_fail(e, "gate_up launch");
-    e = timed(P, 2, [&](const lstk::LaunchTiming *tm) { return lstk::launch_act_quant(sc.act, f, np, s.td, P->aq, st, tm); });
+    e = timed(P, 2, [&](const lstk::LaunchTiming *tm) { return lstk::launch_act_quant(sc.act, f, np, s.td, g.aq, st, tm); });
     if (e != hipSuccess) return hip_fail(e, "act quant launch");
     lstk::GroupedParams dn = gu;
     dn.w0 = s.d_down;
@@ -1024,9 +1056,9 @@ int run_grouped(lstk_pool *P, const Shard &s, const CallScratch &sc, bool fixed,
     dn.stride1 = 0;
     dn.rows = h;
     dn.K = f;
-    dn.xqs = P->aq.qs;
-    dn.xd = P->aq.d;
-    dn.xbh = P->aq.bh;
+    dn.xqs = g.aq.qs;
+    dn.xd = g.aq.d;
+    dn.xbh = g.aq.bh;
     dn.row_div = 1;
     dn.weights = d_weights;
     dn.out = sc.Y;
@@ -1042,9 +1074,9 @@ int run_grouped(lstk_pool *P, const Shard &s, const CallScratch &sc, bool fixed,
     return LSTK_OK;
 }
 
-// fixed != null (lstk_moe_block_noalloc): the scratch comes from the fixed array (a many-token call's work list and its
-// quantized SwiGLU rows from the pool's, laid out for n_batch at creation), and the call takes neither the fused path nor
-// the stage timing (which creates events).
+// fixed != null (lstk_moe_block_noalloc): the scratch comes from the fixed array (nothing of the pool's is written but its
+// error flag; a call whose grouped part does not fit beside the rest takes the GEMV path), and the call takes neither the
+// fused path nor the stage timing (which creates events).
 int run_block(lstk_pool *P, int layer, int mode, const float *d_hnorm, const void *d_gate_inp, int gate_type,
               const int32_t *d_slots, int32_t *d_ids, float *d_weights, const float *d_resid, float *d_out, int T,
               hipStream_t st, const NormIn *norm = nullptr, const CallScratch *fixed = nullptr) {
@@ -1053,7 +1085,7 @@ int run_block(lstk_pool *P, int layer, int mode, const float *d_hnorm, const voi
     const int k = d.n_expert_used;
     if (!fixed && T == 1 && !norm && use_fused(P, s, mode == 1 ? gate_type : lstk::kTypeF16))
         return run_fused(P, s, mode, d_hnorm, d_gate_inp, gate_type, d_slots, d_ids, d_weights, d_resid, d_out, st);
-    const CallScratch sc = fixed ? *fixed : CallScratch{P->xq, P->logits, P->act, P->Y};
+    const CallScratch sc = fixed ? *fixed : CallScratch{P->xq, P->logits, P->act, P->Y, P->grouped};
     auto timed = [&](lstk_pool *pool, int stage, auto &&launch) -> hipError_t {
         return fixed ? launch(nullptr) : ::timed(pool, stage, launch);
     };
@@ -1074,8 +1106,8 @@ int run_block(lstk_pool *P, int layer, int mode, const float *d_hnorm, const voi
     rp.logits = sc.logits;
     rp.qtype = s.tu;
     rp.xq = sc.xq;
-    const bool grouped = use_grouped(P, s, T);
-    rp.xq.bh = grouped ? P->xq.bh : nullptr; // only the grouped kernels read the split group sums
+    const bool grouped = sc.grouped.counts && use_grouped(P, s, T);
+    rp.xq.bh = grouped ? sc.grouped.xbh : nullptr; // only the grouped kernels read the split group sums
     hipError_t e = timed(P, 0, [&](const lstk::LaunchTiming *tm) { return lstk::launch_route(rp, st, tm); });
     if (e != hipSuccess) return hip_fail(e, "route launch");
     const bool fused_topk = mode == 1 && !grouped && T <= lstk::decode_route_max_tokens(); // grouped reads d_ids
@@ -1350,6 +1382,8 @@ int lstk_moe_block_noalloc(lstk_pool *pool, int layer, const float *d_hnorm, con
     if (!pool->noalloc) return fail(LSTK_E_DEVICE, "the fixed scratch has no address on this device");
     CallScratch sc{};
     call_scratch_layout(pool->dims, n_tokens, pool->noalloc, &sc);
+    const int n_bins = (int) pool->shards[pool->layer_shard[layer]].n_slots;
+    if (noalloc_grouped(pool->dims, n_bins, n_tokens)) grouped_scratch(pool->dims, n_tokens, n_bins, pool->noalloc + need, &sc.grouped);
     return run_block(pool, layer, 1, d_hnorm, d_gate_inp, gate_type, nullptr, d_ids, d_weights, d_resid, d_out, n_tokens,
                      static_cast<hipStream_t>(stream), nullptr, &sc);
 }
@@ -1432,6 +1466,20 @@ int lstk_unpack_matrix(int type, int rows, int cols, const void *packed, void *g
     if (!gguf || !packed) return fail(LSTK_E_INVALID, "null argument");
     const int rc = lstk::unpack_matrix(type, rows, cols, packed, gguf);
     return rc == LSTK_OK ? rc : fail(rc, "unsupported type or shape");
+}
+
+int lstk_debug_moe_plan(const lstk_moe_dims *dims, int type_gate, int type_down, int n_slots, int n_tokens, int32_t out[5]) {
+    if (!dims || !out || n_slots < 1 || n_tokens < 1 || dims->n_expert < 1 || dims->n_expert_used < 1 || dims->n_embd < 256 ||
+        dims->n_ff_exp < 256)
+        return fail(LSTK_E_INVALID, "lstk_debug_moe_plan: bad arguments");
+    const bool grouped = takes_grouped(*dims, type_gate, type_gate, type_down, n_slots, n_tokens, grouped_env());
+    const GroupedPlan g = grouped_plan(type_gate, type_down, n_tokens * dims->n_expert_used, dims->n_expert);
+    out[0] = grouped;
+    out[1] = grouped && g.rows;
+    out[2] = grouped ? g.chunk : 0;
+    out[3] = grouped && g.once;
+    out[4] = grouped && noalloc_grouped(*dims, n_slots, n_tokens);
+    return LSTK_OK;
 }
 
 // Test hook: makes the next n host-tier copies fail, to exercise the LSTK_E_IO path.

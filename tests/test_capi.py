@@ -125,6 +125,25 @@ def test_dry_pool_refuses_compute(lstk):
         p.permute(16, 8, 16, 16, 16, n_tokens=1, stream=0)
 
 
+@pytest.mark.parametrize("types", [(8, 8, 8), (12, 12, 12), (10, 10, 11)])
+@pytest.mark.parametrize("h,f,E,k", [(2048, 768, 128, 8), (4096, 1536, 128, 8), (1024, 512, 16, 2)])
+def test_noalloc_groups_only_in_its_own_scratch(lstk, types, h, f, E, k):
+    """lstk_moe_block_noalloc takes the grouped path exactly where the fixed array holds everything that path writes
+    (restated here part by part, 256-byte aligned), so no call needs the pool's scratch."""
+    up = lambda n: (n + 255) // 256 * 256
+    for T in list(range(1, 200)) + [255, 256, 511, 512]:
+        np_ = T * k
+        rows = lambda n, w: [n * w] + 2 * [n * (w // 32) * 4]  # quants, scales, group sums
+        parts = rows(T, h) + [T * E * 4, np_ * f * 4, np_ * h * 4]
+        items = (np_ + 15) // 16 + min(E, np_)
+        parts += [E * 4, (E + 1) * 4, np_ * 4, 64, items * 16] + rows(np_, f) + [np_ * (f // 32) * 4, T * (h // 32) * 4]
+        grouped, rows_k, chunk, once, noalloc = lstk.moe_plan(types, h, f, E, k, T)
+        assert noalloc == (grouped and sum(map(up, parts)) <= 16 << 20), T
+        assert chunk in ((16, 32) if grouped else (0,)) and (grouped or not (rows_k or once))
+    with pytest.raises(lstk.LstkError):
+        lstk.moe_plan(types, h, f, E, k, 0)
+
+
 def test_missing_library_fails_loudly(tmp_path, monkeypatch):
     import importlib
     import localstack_amd

@@ -1,7 +1,8 @@
 """lstk_moe_block_noalloc (the MoE block with its scratch in the library's fixed per-device array)
 against lstk_moe_block on the same pool and inputs, through the C ABI: bit-identical ids, weights and
 outputs on two calls in a row, the second with fewer tokens (the array keeps the first call's
-contents), at the 30B-A3B shape with Q8_0 experts and at a Q4_K shape; and the size limit."""
+contents), at the 30B-A3B shape with Q8_0 experts and at a Q4_K shape; the sizes around the last one whose
+grouped scratch the array holds; and the size limit."""
 import numpy as np
 import pytest
 
@@ -53,6 +54,34 @@ def test_noalloc_block_matches_block(lstk, dev, wtype, h, f, E, k, n_batch, call
         assert torch.equal(w_a, w_b), f"call {i} (T={T}): router weights differ"
         assert torch.isfinite(out_b).all()
         assert torch.equal(out_a, out_b), f"call {i} (T={T}): outputs differ, max {float((out_a - out_b).abs().max())}"
+    store.close()
+
+
+@pytest.mark.parametrize("wtype", (8, 12))
+def test_noalloc_around_the_last_grouped_size(lstk, dev, wtype):
+    """The most tokens the array's grouped scratch allows give lstk_moe_block's bits; one more, and the most tokens the
+    array takes at all, run on the GEMV path and agree to the expert kernels' bar (test_gpu_grouped_rows.py)."""
+    import torch
+    h, f, E, k, n_batch = 2048, 768, 128, 8, 180
+    rng = np.random.default_rng(31 + wtype)
+    types = (wtype,) * 3
+    last = max(T for T in range(1, n_batch + 1) if lstk.moe_plan(types, h, f, E, k, T)[4])
+    assert last < n_batch
+    mats = [synth.experts(rng, wtype, E, r, c, centered=True) for r, c in ((f, h), (f, h), (h, f))]
+    router = torch.from_numpy(synth.router_f16(rng, E, h)).to(dev)
+    store = lstk.ExpertStore(1, h, f, E, k, n_batch, [(types, *mats)])
+    for T in (last, last + 1, n_batch):
+        x, resid = _inputs(torch, dev, rng, T, h)
+        outs = [_outs(torch, dev, T, h, k) for _ in range(2)]
+        for call, o in zip((store.block, store.block_noalloc), outs):
+            call(0, x, router, lstk.TYPE_F16, resid, *o)
+            store.check()
+        (a, ia, wa), (b, ib, wb) = outs
+        print(f"noalloc T={T} type={wtype}: max {float((a - b).abs().max() / (a - resid).abs().max()):.2e}", flush=True)
+        assert torch.equal(ia, ib) and torch.equal(wa, wb)
+        if T == last:
+            assert torch.equal(a, b)
+        assert float((a - b).abs().max()) <= 2e-3 * float((a - resid).abs().max())
     store.close()
 
 
