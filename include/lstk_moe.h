@@ -167,7 +167,9 @@ int lstk_moe_route(lstk_pool *pool, int layer, const float *d_hnorm, int n_token
  * d_out may alias d_resid.
  * From some tokens on (9 with Q4_K experts, up to 32 by format and expert size; LSTK_GROUPED_MIN_TOKENS in the
  * environment overrides the threshold) the call takes the grouped path: a stable permutation of the pairs by
- * expert, then expert products on the matrix cores over chunks of 16 or 32 pairs. */
+ * expert, then expert products on the matrix cores over chunks of 16 or 32 pairs.
+ * A token's slots are meant to be distinct. A slot in more than n_tokens pairs is reported by lstk_pool_check as an id
+ * out of range is, except in all-Q4_K calls of at least 64 tokens (or under LSTK_GROUPED_MIN_TOKENS), which take it. */
 int lstk_moe_ffn(lstk_pool *pool, int layer, const float *d_hnorm, const int32_t *d_slots, const float *d_weights,
                  const float *d_resid, float *d_out, int n_tokens, lstk_stream_t stream);
 

@@ -1002,6 +1002,15 @@ size_t call_scratch_layout(const lstk_moe_dims &d, int T, uint8_t *base, CallScr
     return off;
 }
 
+// The most pairs an expert may have before lstk_pool_check reports a repeated id (0: no report). The GEMV kernels hold an
+// expert's pairs in a list of T and report more, so a grouped call does too. All-Q4_K calls of 64 tokens, or of any size
+// under LSTK_GROUPED_MIN_TOKENS, have always taken repeated ids (every pair counts), and still do.
+constexpr int kRepeatedIdsFrom = 64;
+int repeat_limit(int tg, int td, int T, int env) {
+    const bool q4 = tg == lstk::kTypeQ4_K && td == lstk::kTypeQ4_K;
+    return q4 && (env > 0 || T >= kRepeatedIdsFrom) ? 0 : T;
+}
+
 // Whether the fixed array holds the grouped part of a call of T tokens behind the rest.
 bool noalloc_grouped(const lstk_moe_dims &d, int n_bins, int T) {
     return call_scratch_layout(d, T, nullptr, nullptr) + grouped_scratch(d, T, n_bins, nullptr, nullptr) <= kNoAllocBytes;
@@ -1021,7 +1030,7 @@ int run_grouped(lstk_pool *P, const Shard &s, const CallScratch &sc, bool fixed,
     const int max_items = lstk::grouped_max_items(np, (int) s.n_slots, chunk);
     const GroupedScratch &g = sc.grouped;
     lstk::PermuteParams pp{bins, np, (int) s.n_slots, chunk, g.counts, g.offsets, g.perm,
-                           g.items, g.n_items, P->err, T < 64 || s.tg != lstk::kTypeQ4_K || s.td != lstk::kTypeQ4_K ? T : 0};
+                           g.items, g.n_items, P->err, repeat_limit(s.tg, s.td, T, P->grouped_min_tokens)};
     hipError_t e = timed(P, 0, [&](const lstk::LaunchTiming *tm) { return lstk::launch_permute(pp, st, tm); });
     if (e != hipSuccess) return hip_fail(e, "permute launch");
     lstk::GroupedParams gu{};

@@ -129,3 +129,32 @@ def test_q8_0_sums_are_as_close_to_64_bits_as_the_gemv_paths(lstk, dev, E):
     print(f"[Q8_0 K={f} E={E}] error against 64 bits: many tokens {err[0]:.3e}, GEMV {err[1]:.3e}", flush=True)
     assert err[1] < 2e-7, "the quantized rows are not the integers this test assumes"
     assert err[0] <= 1.05 * err[1]
+
+
+@pytest.mark.parametrize("types,T,env,taken", [
+    ((12, 12, 12), 63, None, False), ((12, 12, 12), 64, None, True), ((12, 12, 12), 20, "16", True), ((12, 12, 12), 15, "16", False),
+    ((8, 8, 8), 64, None, False), ((8, 8, 8), 64, "16", False), ((12, 12, 14), 64, None, False), ((12, 12, 14), 64, "16", False),
+], ids=str)
+def test_repeated_ids_are_reported_or_taken_as_before(orc, lstk, dev, monkeypatch, types, T, env, taken):
+    """Every token names expert 3 twice (2 T pairs of one expert): reported by check() as on the GEMV path, except in
+    all-Q4_K calls of 64 tokens or under the threshold's override, which count every pair."""
+    import torch
+    h, f, E, k = 256, 512, 16, 2
+    if env:
+        monkeypatch.setenv("LSTK_GROUPED_MIN_TOKENS", env)
+    rng = np.random.default_rng(T)
+    mats = [synth.experts(rng, t, E, r, c, centered=True) for t, (r, c) in zip(types, ((f, h), (f, h), (h, f)))]
+    x, resid = synth.activations(rng, T, h), synth.activations(rng, T, h)
+    ids, w = np.full((T, k), 3, np.int32), rng.uniform(0.1, 0.9, (T, k)).astype(np.float32)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    store = lstk.ExpertStore(1, h, f, E, k, T, [(types, *mats)])
+    out = torch.full((T, h), np.nan, dtype=torch.float32, device=dev)
+    store.ffn(0, d(x), d(ids), d(w), d(resid), out)
+    if taken:
+        store.check()
+        ref = orc.moe_ffn(x, ids, w, resid, *(m.reshape(E, -1) for m in mats), types, f)
+        assert np.abs(out.cpu().numpy() - ref).max() <= FFN_TOL * np.abs(ref - resid).max()
+    else:
+        with pytest.raises(lstk.LstkError, match="repeated within one token"):
+            store.check()
+    store.close()
