@@ -206,6 +206,44 @@ __device__ __forceinline__ int sext_byte(unsigned v, int i) {
     return s;
 }
 
+// Q8_0 rows with an infinite scale (no quantizer writes one): d_w I is +-inf there, but the fma with -1.5 2^23 d_w above
+// gives inf - inf. Sums that came out NaN are therefore formed again from plain products, as the GEMV kernels form them
+// (and stay NaN where a scale or activation is, or for 0 inf); the others keep their values.
+template <int MT, int CH>
+__device__ __forceinline__ void rows_plain_q8(const RLds &L, int K, const uint8_t *w0, const uint8_t *w1, f32x4 (&acc)[2][MT]) {
+    constexpr int C = chunks_of(kTypeQ8_0);
+    const unsigned lane = threadIdx.x % kWave, r = lane % 16, kg = lane / 16;
+    f32x4 sum[2][MT];
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) sum[t][mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+    for (int b = 0; b < K / 32; b++) {
+        Acts<kTypeQ8_0, MT> x;
+        load_acts<kTypeQ8_0, MT, CH>(x, L, K, b / 8, b % 8);
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const uint8_t *w = (t ? w1 : w0) + (size_t) (b / 8) * (C * 256);
+            const float d = h2f(*reinterpret_cast<const uint16_t *>(w + r * 16 + 2 * (b % 8)));
+            const uint2 q = load_q<kTypeQ8_0, false>(w, b % 8);
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) {
+                const f32x4 dx = *reinterpret_cast<const f32x4 *>(L.dx + b * CH + 16 * mt + 4 * kg);
+                const i32x4 I = mfma8(x.a[0][mt], q, i32x4{0, 0, 0, 0});
+#pragma unroll
+                for (int i = 0; i < 4; i++) sum[t][mt][i] += (float) I[i] * (d * dx[i]);
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[t][mt][i] = acc[t][mt][i] != acc[t][mt][i] ? sum[t][mt][i] : acc[t][mt][i];
+}
+
 // The whole K of the wavefront's two tiles (rows at w0, w1) against the item's rows: acc[tile][mt][i] = token
 // 16 mt + 4 (lane / 16) + i of the item, row lane % 16 of the tile. q / h hold super-block 0. A block's quants are
 // requested for the next super-block as soon as they have been multiplied, into the same registers, so every load
@@ -411,6 +449,16 @@ __device__ __forceinline__ void rows_products(const RLds &L, int K, const uint8_
     };
     for (int sb = 0; sb + 1 < nsb; sb++) super_block(sb, std::true_type{});
     super_block(nsb - 1, std::false_type{});
+    if constexpr (WT == kTypeQ8_0) {
+        bool nan = false;
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) nan |= acc[t][mt][i] != acc[t][mt][i];
+        if (__ballot(nan) != 0ull) rows_plain_q8<MT, CH>(L, K, w0, w1, acc);
+    }
 }
 
 // Work-group b -> (item, row block): XCD x = b % 8 takes the items [x per, (x + 1) per), all row blocks of an item before

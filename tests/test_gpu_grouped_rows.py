@@ -158,3 +158,36 @@ def test_repeated_ids_are_reported_or_taken_as_before(orc, lstk, dev, monkeypatc
         with pytest.raises(lstk.LstkError, match="repeated within one token"):
             store.check()
     store.close()
+
+
+@pytest.mark.parametrize("E", (2, 16), ids=("32-pair items", "16-pair items"))
+def test_q8_0_infinite_scales_as_on_the_gemv_path(lstk, dev, E):
+    """Down rows with a block whose fp16 scale is +-inf or NaN, in a few rows: the many-token call gives the infinities and
+    NaN that calls of 8 tokens (GEMV kernels) give, and every other output to the f32 order of the sums."""
+    import torch
+    h, f, k, T = 512, 1024, 1, 64
+    rng = np.random.default_rng(17)
+    mats = [synth.experts(rng, 8, E, r, c) for r, c in ((f, h), (f, h), (h, f))]
+    blocks = mats[2].reshape(E, h, f // 32, 34)
+    for row, blk, v in ((0, 0, np.inf), (17, 31, -np.inf), (18, 5, np.inf), (100, 9, np.nan), (511, 30, -np.inf)):
+        blocks[:, row, blk, :2] = np.array([v], np.float16).view(np.uint8)
+    blocks[:, 18, 5, 2:] = 0  # 0 inf
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    x = synth.activations(rng, T, h)
+    store = lstk.ExpertStore(1, h, f, E, k, T, [((8, 8, 8), *mats)])
+    out = []
+    for step in (T, 8):
+        o = torch.zeros(T, h, device=dev)
+        for t in range(0, T, step):
+            store.ffn(0, d(x[t:t + step]), torch.zeros(step, k, dtype=torch.int32, device=dev), torch.ones(step, k, device=dev),
+                      torch.zeros(step, h, device=dev), o[t:t + step])
+        store.check()
+        out.append(o.cpu().numpy())
+    store.close()
+    many, few = out
+    assert lstk.moe_plan((8, 8, 8), h, f, E, k, T)[:3] == (True, True, 32 if E == 2 else 16)
+    assert np.isinf(few[:, [0, 17, 511]]).all() and np.isnan(few[:, [18, 100]]).all()
+    fin = np.isfinite(few)
+    assert fin.sum() == T * (h - 5)
+    np.testing.assert_array_equal(many[~fin], few[~fin])
+    assert np.abs(many[fin] - few[fin]).max() <= FFN_TOL * np.abs(few[fin]).max()
