@@ -12,6 +12,7 @@
 
 #include "formats.h"
 #include "kernels.h"
+#include "once.h"
 
 namespace lstk {
 
@@ -677,6 +678,14 @@ inline bool pick_split(int nsb, int *S, int *G) {
 
 // gate_up additionally needs 128 % G == 0 (rows per work-group = 128 / G).
 inline bool pick_split_gate_up(int nsb, int *S, int *G) { return pick_split(nsb, S, G) && 128 % *G == 0; }
+
+// Lets `kernel` take up to `bytes` of dynamic LDS (gfx950 has 160 KiB per CU; the default limit is 64) on the current
+// device. The limit is an attribute of a device's own copy of the kernel, so every device is asked once.
+inline hipError_t allow_dynamic_lds(const void *kernel, size_t bytes, std::atomic<uint64_t> &done) {
+    int device = 0;
+    if (const hipError_t e = hipGetDevice(&device); e != hipSuccess) return e;
+    return once_per_device(done, device, [&] { return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int) bytes); });
+}
 
 // A launch on `st`; with `tm` set, the launch records its own start / stop timestamps.
 template <typename K, typename... A>

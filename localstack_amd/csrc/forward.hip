@@ -1769,9 +1769,9 @@ hipError_t launch_attn_hd(const AttnParams &P, hipStream_t st, const LaunchTimin
         if (P.rb_rows == 64 && !P.rope_in) {
             if (attn_in_split(P)) {
                 constexpr size_t lds = sizeof(AttnSplitLds<HD>);
-                static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_split_kernel<HD>),
-                                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
-                if (allowed != hipSuccess) return allowed;
+                static std::atomic<uint64_t> allowed{0};
+                if (const hipError_t e = allow_dynamic_lds(reinterpret_cast<const void *>(&attn_split_kernel<HD>), lds, allowed); e != hipSuccess)
+                    return e;
                 return launch(attn_split_kernel<HD>, grid, dim3(kAsWaves * kWave), lds, st, tm, P);
             }
             return launch(attn_rows_kernel<HD>, grid, block, 0, st, tm, P);

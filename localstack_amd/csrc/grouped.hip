@@ -583,23 +583,11 @@ hipError_t launch_permute(const PermuteParams &P, hipStream_t st, const LaunchTi
     return launch(permute_kernel, dim3(1), dim3(kPermThreads), 0, st, tm, P);
 }
 
-// The grouped kernels take more than 64 KiB of dynamic LDS (gfx950 has 160 KiB per CU).
-hipError_t allow_lds() {
-    static hipError_t e = [] {
-        hipError_t r = hipFuncSetAttribute(reinterpret_cast<const void *>(&gate_up_grouped_kernel),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int) kGLdsBytes);
-        if (r == hipSuccess)
-            r = hipFuncSetAttribute(reinterpret_cast<const void *>(&down_grouped_kernel),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int) kGLdsBytes);
-        return r;
-    }();
-    return e;
-}
-
 hipError_t launch_gate_up_grouped(const GroupedParams &P, int max_items, hipStream_t st, const LaunchTiming *tm) {
     if (max_items <= 0) return hipSuccess;
     if (!P.xbh) return hipErrorInvalidValue;
-    if (const hipError_t e = allow_lds(); e != hipSuccess) return e;
+    static std::atomic<uint64_t> allowed{0};
+    if (const hipError_t e = allow_dynamic_lds(reinterpret_cast<const void *>(&gate_up_grouped_kernel), kGLdsBytes, allowed); e != hipSuccess) return e;
     const int per = (max_items + kXcds - 1) / kXcds;
     return launch(gate_up_grouped_kernel, dim3(kXcds * per * (P.rows / 64)), dim3(kGThreads), kGLdsBytes, st, tm, P);
 }
@@ -607,7 +595,8 @@ hipError_t launch_gate_up_grouped(const GroupedParams &P, int max_items, hipStre
 hipError_t launch_down_grouped(const GroupedParams &P, int max_items, hipStream_t st, const LaunchTiming *tm) {
     if (max_items <= 0) return hipSuccess;
     if (!P.xbh) return hipErrorInvalidValue;
-    if (const hipError_t e = allow_lds(); e != hipSuccess) return e;
+    static std::atomic<uint64_t> allowed{0};
+    if (const hipError_t e = allow_dynamic_lds(reinterpret_cast<const void *>(&down_grouped_kernel), kGLdsBytes, allowed); e != hipSuccess) return e;
     const int per = (max_items + kXcds - 1) / kXcds;
     return launch(down_grouped_kernel, dim3(kXcds * per * (P.rows / 128)), dim3(kGThreads), kGLdsBytes, st, tm, P);
 }

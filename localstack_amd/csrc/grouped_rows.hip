@@ -532,9 +532,9 @@ __global__ __launch_bounds__(NW *kWave, WT == kTypeKQ8 ? (NW == 8 ? 2 : 3) : 4) 
 template <int WT, bool MINS, int MT, bool DOWN, int NW, bool NT>
 hipError_t launch_rows_n(const GroupedParams &P, int max_items, hipStream_t st, const LaunchTiming *tm) {
     const size_t lds = r_lds<WT>(16 * MT, P.K, nullptr, nullptr);
-    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void *>(&rows_kernel<WT, MINS, MT, DOWN, NW, NT>),
-                                                          hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    if (allowed != hipSuccess) return allowed;
+    static std::atomic<uint64_t> allowed{0};
+    const void *kernel = reinterpret_cast<const void *>(&rows_kernel<WT, MINS, MT, DOWN, NW, NT>);
+    if (const hipError_t e = allow_dynamic_lds(kernel, 160 * 1024, allowed); e != hipSuccess) return e;
     const int per = (max_items + kRXcds - 1) / kRXcds;
     return launch(rows_kernel<WT, MINS, MT, DOWN, NW, NT>, dim3(kRXcds * per * (P.rows / (DOWN ? 32 * NW : 16 * NW))), dim3(NW * kWave), lds, st, tm, P);
 }
