@@ -139,6 +139,8 @@ bool attn_supported(int hd);
 // n_kv and n_cells. The partial rows (T * n_head * n_chunk when n_chunk > 1) stay below
 // attn_part_rows(n_batch, n_head).
 void attn_plan(AttnParams &P);
+// Whether a planned launch takes attn_split_kernel (its partial rows' maxima are exponents of 2).
+bool attn_in_split(const AttnParams &P);
 size_t attn_part_rows(int n_batch, int n_head);
 
 hipError_t launch_rmsnorm(const NormParams &P, hipStream_t st, const LaunchTiming *tm);

@@ -1045,7 +1045,7 @@ __global__ __launch_bounds__(NW *kWave) void attn1_kernel(AttnParams P) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// Attention of 64-row blocks (steps of 8 to 63 tokens at 8 query heads per KV head): wavefront w owns query rows row0 + 16 w .. + 15
+// Attention of 64-row blocks (steps of many tokens; long chunks: attn_split_kernel): wavefront w owns query rows row0 + 16 w .. + 15
 // over the whole chunk and runs them from registers to registers as attn1_kernel does (S^T = K Q^T puts
 // a row's scores in that row's lanes, the online softmax stays there, O^T += V^T P^T with P as fp16
 // hi + lo). The K and V fragments of each 64-cell block (and its cell-table entries) are loaded once
@@ -1053,12 +1053,13 @@ __global__ __launch_bounds__(NW *kWave) void attn1_kernel(AttnParams P) {
 // wavefronts read them; the next live block's loads are in flight while a block is multiplied. Two
 // barriers per 64-cell block; no score or probability goes through LDS.
 // ------------------------------------------------------------------------------------------------
-template <int HD>
+template <int HD, bool SKIP>
 __global__ __launch_bounds__(kAtBlock) void attn_rows_kernel(AttnParams P) {
     constexpr int NK = HD / 16;
     __shared__ __align__(16) half4v s_k[4][NK][kWave];
     __shared__ __align__(16) half4v s_v[4][NK][kWave];
     __shared__ __align__(16) int s_cs[kFaCells], s_cp[kFaCells];
+    __shared__ uint8_t s_live[SKIP ? kAttnMaxPasses : 1];
     const int tid = threadIdx.x, w = tid / kWave, l = tid & (kWave - 1), lr = l & 15, lq = l >> 4;
     const int grp = P.n_head / P.n_kv;
     const int g = blockIdx.x % P.n_kv, rest = blockIdx.x / P.n_kv;
@@ -1085,6 +1086,22 @@ __global__ __launch_bounds__(kAtBlock) void attn_rows_kernel(AttnParams P) {
         const int ct = min(b0 + 16 * w + (l & 15), P.kv_size - 1);
         ctr = l < 16 ? P.cell_seq[ct] : P.cell_pos[ct];
     };
+    // A step of many tokens skips the chunk's passes that hold no cell of the sequence (attn_kernel's map)
+    const bool skip = SKIP && n_pass <= kAttnMaxPasses;
+    if (skip) {
+        for (int p0 = 0; p0 < n_pass; p0 += 8 * (kAtBlock / kWave)) {
+            int cs[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) cs[u] = P.cell_seq[min(begin + (p0 + u * (kAtBlock / kWave) + w) * kFaCells + l, P.kv_size - 1)];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const int pass = p0 + u * (kAtBlock / kWave) + w;
+                const bool mine = cs[u] == P.seq && begin + pass * kFaCells + l < end;
+                const bool any = __ballot(mine) != 0ull;
+                if (l == 0 && pass < n_pass) s_live[pass] = any ? 1 : 0;
+            }
+        }
+    }
     half4v qb[NK];
     const uint16_t *q = P.q + ((size_t) t * P.n_head + h) * HD;
 #pragma unroll
@@ -1092,7 +1109,13 @@ __global__ __launch_bounds__(kAtBlock) void attn_rows_kernel(AttnParams P) {
         const half4v v = ld_half4(q + ks * 16 + 4 * lq);
         qb[ks] = on ? v : half4v{0, 0, 0, 0};
     }
-    int p = 0;
+    __syncthreads(); // the skip map
+    auto next_live = [&](int p) {
+        if (skip)
+            while (p < n_pass && !s_live[p]) p++;
+        return p;
+    };
+    int p = next_live(0);
     load_block(begin + min(p, n_pass - 1) * kFaCells);
     float m_run = -INFINITY, l_run = 0.0f;
     f32x4v o[NK];
@@ -1108,7 +1131,7 @@ __global__ __launch_bounds__(kAtBlock) void attn_rows_kernel(AttnParams P) {
         if (l < 16) s_cs[16 * w + l] = ctr;
         else if (l < 32) s_cp[16 * w + l - 16] = ctr;
         __syncthreads();
-        const int pn = p + 1;
+        const int pn = next_live(p + 1);
         load_block(begin + min(pn, n_pass - 1) * kFaCells); // unconditional: the last block again past the end
         // the block's four 16-cell groups together: S^T of each (four independent product chains), one
         // softmax step over the 64 cells, then O^T += V^T P^T over the groups (eight chains, one per dim tile)
@@ -1193,8 +1216,8 @@ __global__ __launch_bounds__(kAtBlock) void attn_rows_kernel(AttnParams P) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// Prompt attention (steps of many tokens in 64-row blocks). The work-group's eight wavefronts split the cells, not the
-// rows: a wavefront takes every eighth 16-cell unit of the chunk for all 64 rows, with its K and V fragments loaded
+// Prompt attention (steps of many tokens in 64-row blocks with long chunks, attn_in_split). The work-group's eight
+// wavefronts split the cells, not the rows: a wavefront takes every eighth 16-cell unit of the chunk for all 64 rows, with its K and V fragments loaded
 // straight from the cache into registers (the cache layout is the operand layout) and the rows' Q fragments read from
 // LDS. Each keeps a running maximum, sum and output of all 64 rows for its own cells, so nothing is exchanged and no
 // barrier is met until the end, where the eight partial rows are summed through LDS. A prompt's launch is about one
@@ -1750,8 +1773,19 @@ hipError_t launch_rope(const RopeParams &P, hipStream_t st, const LaunchTiming *
     return launch(rope_kernel, dim3(P.T, P.n_head + 2 * P.n_kv), dim3(kWave), 0, st, tm, P);
 }
 
-// Launches of attn_split_kernel: many-token steps in 64-row blocks (head size 256 would need 128 KB of fragments a block).
-bool attn_in_split(const AttnParams &P) { return P.T >= kAttnSkipMinT && P.rb_rows == 64 && !P.rope_in && P.hd <= 128; }
+// Launches of attn_split_kernel: many-token steps in 64-row blocks (head size 256 would need 128 KB of fragments a block)
+// with long chunks. Its work-groups take 156 KB of LDS, so a CU holds one, and eight wavefronts share 16 cells at a time:
+// a chunk of 64 or 128 cells leaves most of them idle, and past one work-group per CU the next ones wait for a whole
+// work-group to end, where four of attn_rows_kernel's share a CU. attn_rows_kernel / attn_split_kernel, us a launch with
+// its combine:
+//   up to 256 work-groups: chunks of 64 cells 11.2 / 13.0, 128 16.8 / 17.6, 192 19.7 / 18.3, 256 23.4 / 20.6, 512 35.4 / 25.9
+//   more, head size 128: 64 22.4 / 30.9, 192 34.5 / 39.8, 320 37.6 / 39.5, 384 40.7 / 40.3 and 37.1 / 41.8, 512 45.8 / 44.2 and
+//     45.1 / 46.7, 576 52.0 / 47.2, 768 60.9 / 55.8, 1024 75.3 / 61.2
+//   more, head size 64: 320 30.3 / 30.4, 448 36.2 / 38.0, 704 50.8 / 53.6, 768 46.8 / 39.9 and 56.4 / 51.7, 960 54.4 / 46.1
+bool attn_in_split(const AttnParams &P) {
+    if (P.T < kAttnSkipMinT || P.rb_rows != 64 || P.rope_in || P.hd > 128) return false;
+    return P.chunk >= (P.n_kv * P.n_chunk * P.n_rowblk <= kAttn1Wgs ? 192 : P.hd == 64 ? 768 : 576);
+}
 
 template <int HD>
 hipError_t launch_attn_hd(const AttnParams &P, hipStream_t st, const LaunchTiming *tm) {
@@ -1774,7 +1808,8 @@ hipError_t launch_attn_hd(const AttnParams &P, hipStream_t st, const LaunchTimin
                     return e;
                 return launch(attn_split_kernel<HD>, grid, dim3(kAsWaves * kWave), lds, st, tm, P);
             }
-            return launch(attn_rows_kernel<HD>, grid, block, 0, st, tm, P);
+            if (P.T >= kAttnSkipMinT) return launch(attn_rows_kernel<HD, true>, grid, block, 0, st, tm, P);
+            return launch(attn_rows_kernel<HD, false>, grid, block, 0, st, tm, P);
         }
     }
     // steps of many tokens (prompts): the instantiation that skips passes with no cell of the sequence

@@ -810,13 +810,11 @@ int lstk_model_debug_options(lstk_model *model, int flags) {
     return LSTK_OK;
 }
 
-int lstk_debug_attn_plan(int n_tokens, int n_head, int n_kv, int head_dim, int kv_size, int n_cells, int cell_begin,
-                         int rope_in, int32_t out[6]) {
-    if (!out || n_tokens < 1 || n_head < 1 || n_kv < 1 || n_head % n_kv || !lstk::attn_supported(head_dim) ||
-        kv_size < 32 || kv_size % 32 || n_cells < 1 || n_cells > kv_size || cell_begin < 0 || cell_begin >= n_cells ||
-        cell_begin % 64)
-        return set_error(LSTK_E_INVALID, "lstk_debug_attn_plan: bad arguments");
-    lstk::AttnParams ap{};
+static int planned(int n_tokens, int n_head, int n_kv, int head_dim, int kv_size, int n_cells, int cell_begin, int rope_in,
+                   lstk::AttnParams &ap) {
+    if (n_tokens < 1 || n_head < 1 || n_kv < 1 || n_head % n_kv || !lstk::attn_supported(head_dim) || kv_size < 32 ||
+        kv_size % 32 || n_cells < 1 || n_cells > kv_size || cell_begin < 0 || cell_begin >= n_cells || cell_begin % 64)
+        return set_error(LSTK_E_INVALID, "attention plan: bad arguments");
     ap.T = n_tokens;
     ap.n_head = n_head;
     ap.n_kv = n_kv;
@@ -826,12 +824,31 @@ int lstk_debug_attn_plan(int n_tokens, int n_head, int n_kv, int head_dim, int k
     ap.cell_begin = cell_begin;
     ap.rope_in = rope_in ? 1 : 0;
     lstk::attn_plan(ap);
+    return LSTK_OK;
+}
+
+int lstk_debug_attn_plan(int n_tokens, int n_head, int n_kv, int head_dim, int kv_size, int n_cells, int cell_begin,
+                         int rope_in, int32_t out[6]) {
+    if (!out) return set_error(LSTK_E_INVALID, "null argument");
+    lstk::AttnParams ap{};
+    const int rc = planned(n_tokens, n_head, n_kv, head_dim, kv_size, n_cells, cell_begin, rope_in, ap);
+    if (rc != LSTK_OK) return rc;
     out[0] = ap.rb_rows;
     out[1] = ap.n_rowblk;
     out[2] = ap.chunk;
     out[3] = ap.n_chunk;
     out[4] = ap.rope_in;
     out[5] = n_kv * ap.n_chunk * ap.n_rowblk;
+    return LSTK_OK;
+}
+
+int lstk_debug_attn_split(int n_tokens, int n_head, int n_kv, int head_dim, int kv_size, int n_cells, int cell_begin,
+                          int32_t *split) {
+    if (!split) return set_error(LSTK_E_INVALID, "null argument");
+    lstk::AttnParams ap{};
+    const int rc = planned(n_tokens, n_head, n_kv, head_dim, kv_size, n_cells, cell_begin, 0, ap);
+    if (rc != LSTK_OK) return rc;
+    *split = lstk::attn_in_split(ap) ? 1 : 0;
     return LSTK_OK;
 }
 

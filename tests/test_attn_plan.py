@@ -52,6 +52,14 @@ def plan(T, n_head, n_kv, n_cells, target=512, rope_in=False, cell_begin=0, hd=1
     return rb_rows, n_rowblk, chunk, n_chunk, rope_in
 
 
+def split(T, n_head, n_kv, n_cells, target=512, cell_begin=0, hd=128):
+    """attn_in_split (forward.hip): whether a planned launch without RoPE splits the cells over its wavefronts."""
+    rb_rows, n_rowblk, chunk, n_chunk, _ = plan(T, n_head, n_kv, n_cells, target, False, cell_begin, hd)
+    if T < 64 or rb_rows != 64 or hd > 128:
+        return False
+    return chunk >= (192 if n_kv * n_rowblk * n_chunk <= A1_WGS else 768 if hd == 64 else 576)
+
+
 def part_rows(n_batch, n_head):
     return 32768 + n_batch * n_head  # attn_part_rows
 
@@ -174,6 +182,9 @@ def test_replayed_plan_is_the_library_plan(lstk):
                             assert got[:5] == want, (n_head, kv_size, n_cells, cell_begin, T, rope)
                             assert got[5] == n_kv * want[1] * want[3]
                             cases += 1
+                        if T > 1:
+                            assert lstk.attn_split(T, n_head, n_kv, hd, kv_size, n_cells, cell_begin) == \
+                                split(T, n_head, n_kv, n_cells, 512, cell_begin, hd), (n_head, n_cells, cell_begin, T)
     assert cases > 1000
     with pytest.raises(lstk.LstkError):
         lstk.attn_plan(1, 32, 4, 128, 1000, 256)  # kv_size not a multiple of 32
@@ -232,6 +243,20 @@ def test_rope_in_keeps_single_pass_chunks():
     assert plan(32, 32, 4, 4352)[2] == 3 * 64
     assert plan(512, 32, 4, 512)[2:4] == (8 * 64, 1)  # a 512-token prompt: 64 row blocks x 4 KV heads, one chunk
     assert plan(64, 32, 4, 4352)[2:4] == (5 * 64, 14)  # 64 tokens: 8 row blocks x 4 KV heads, several chunks
+
+
+def test_short_chunks_keep_the_row_split(lstk):
+    """attn_split_kernel (one work-group per CU) only where it measured faster: a 512-token prompt of the 30B shape at any
+    context and long contexts of shorter steps, but not 64 .. 256 tokens at a short context, whose 64- to 192-cell chunks took
+    28 .. 39 us there against 19 .. 34 us."""
+    ask = lambda T, ctx, heads=(32, 4), hd=128: lstk.attn_split(T, *heads, hd, 65536, (ctx + T + 255) // 256 * 256)
+    assert all(ask(512, c) for c in (0, 192, 512, 2048, 4000, 16000))
+    assert not any(ask(T, c) for T in (64, 80, 128, 200, 256, 384) for c in (0, 192, 512))
+    assert not any(ask(T, 2048) for T in (64, 96, 128)) and ask(384, 2048) and ask(256, 4000) and ask(64, 16000)
+    assert not any(ask(T, c, (4, 2), 64) for T in (64, 256, 512) for c in (0, 512, 2048)) and ask(512, 16000, (4, 2), 64)
+    assert not ask(512, 4000, (16, 2), 256)  # head size 256 has no such kernel
+    with pytest.raises(lstk.LstkError):
+        lstk.attn_split(64, 32, 4, 128, 1000, 256)
 
 
 def softmax_passes(s, T_rows, pass_cells=FA_CELLS):
