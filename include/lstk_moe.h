@@ -165,8 +165,8 @@ int lstk_moe_route(lstk_pool *pool, int layer, const float *d_hnorm, int n_token
  * the weight type (Q8_0 for Q8_0, Q8_K for Q4_K), and so is the SwiGLU output before down.
  * d_slots holds slot numbers from lstk_pool_acquire (streaming) or expert ids (resident).
  * d_out may alias d_resid.
- * From some tokens on (9 with Q4_K experts, up to 32 by format and expert size; LSTK_GROUPED_MIN_TOKENS in the
- * environment overrides the threshold) the call takes the grouped path: a stable permutation of the pairs by
+ * From some tokens on (by format, expert size, and pairs in all and per expert: at 128 experts, 8 used, 9 tokens with
+ * Q4_K experts and 32 with Q8_0; LSTK_GROUPED_MIN_TOKENS in the environment overrides it) the call takes the grouped path: a stable permutation of the pairs by
  * expert, then expert products on the matrix cores over chunks of 16 or 32 pairs.
  * A token's slots are meant to be distinct. A slot in more than n_tokens pairs is reported by lstk_pool_check as an id
  * out of range is, except in all-Q4_K calls of at least 64 tokens (or under LSTK_GROUPED_MIN_TOKENS), which take it. */

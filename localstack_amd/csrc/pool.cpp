@@ -853,20 +853,32 @@ int check_call(lstk_pool *P, int layer, int T) {
     return LSTK_OK;
 }
 
-// The matrix-core path of many-token calls: from how many tokens on a call takes it (LSTK_GROUPED_MIN_TOKENS overrides).
-// It costs two launches more than the GEMV path (permute, SwiGLU quantization) and wins where experts have several
-// pairs, which skewed routing brings early. Measured on one layer, GEMV path against this one, us:
-//   Q4_K gate, up and down: 30B shape 9 tokens 51 / 50 evenly routed and 45 / 40 Zipf(1.1)-routed, 12 61 / 56 and 53 / 40, 24
-//     80 / 68 and 87 / 43, 40 114 / 91; 235B shape 12 218 / 180.
-//   Q4_K gate and up, another k-quant down: 12 70 / 64, 17 83 / 75 and 73 / 44.
-//   KQ8 gate and up (Q2_K + Q3_K): 12 89 / 94 and 80 / 51, 17 107 / 112 and 106 / 55, 24 125 / 123 and 135 / 54.
-//   Q8_0: 24 101 / 112 and 86 / 61, 32 118 / 126 and 114 / 59, 48 147 / 140.
+// The matrix-core path of many-token calls: when a call takes it (LSTK_GROUPED_MIN_TOKENS overrides: from that many tokens).
+// It costs two launches more than the GEMV path (permute, SwiGLU quantization; some 8 us) and wins where experts have
+// several pairs, which skewed routing brings early; evenly routed calls draw the lines. Three of them, all to be met:
+//   tokens, as measured at 128 experts, 8 used, h 2048, f 768. GEMV path against this one, us a layer, even and Zipf(1.1):
+//     Q4_K gate, up and down: 6 44 / 47 and 36 / 38, 8 49 / 49 and 40 / 40, 9 51 / 50 and 43 / 40, 12 59 / 56 and 51 / 41, 24 80 / 71
+//     Q4_K gate and up, another k-quant down: 8 56 / 56 and 46 / 43, 12 69 / 66 and 57 / 44, 17 80 / 75 and 71 / 45
+//     KQ8 gate and up (Q2_K + Q3_K): 12 92 / 88 and 76 / 54, 17 107 / 102 and 92 / 56, 24 123 / 112 and 117 / 63
+//     Q8_0: 16 86 / 90 and 69 / 52, 24 102 / 101 and 90 / 60, 32 118 / 113 and 110 / 64, 48 150 / 126 and 152 / 77
+//   pairs, which pay for the launches: 64, or 96 for Q4_K experts below two million weights (fewer experts or fewer used
+//     each, even routing). 16 experts, 2 used: Q4_K 18 pairs 27 / 34, 48 35 / 35, 64 37 / 35; Q4_K + Q6_K 24 32 / 36, 64 39 / 37;
+//     Q2_K + Q3_K 34 39 / 40; Q8_0 48 38 / 38, 64 40 / 39. 8 experts, 1 used: Q4_K 32 31 / 34, 48 35 / 35. 32 experts of h 1024,
+//     f 512, 4 used: Q4_K 36 27 / 31, 68 31 / 32, 96 32 / 32
+//   pairs per expert (most experts then have a few): 1/2 with Q4_K experts, 3/4 with other k-quants among them, 3/2 with
+//     Q8_0 among them. 128 experts of h 1024, f 768, 1 used: Q4_K 0.38 32 / 37, Q4_K + Q6_K 0.5 40 / 41, Q2_K + Q3_K 0.5 47 / 48, Q8_0 0.5
+//     42 / 45, 0.75 58 / 60; 256 experts, 8 used: Q4_K 0.28 43 / 45, 0.38 51 / 52
 // Experts below a million weights (the tiny shapes) are cheap either way, so their calls keep the fewer launches up to
-// 31 tokens (h 256, f 512, 8 experts, Q8_0: 17 tokens 28 / 35, 32 40 / 34).
-int grouped_from(int tg, int td, int h, int f) {
-    if ((long) 3 * h * f < 1000000 || tg == lstk::kTypeQ8_0) return 32;
-    if (tg != lstk::kTypeQ4_K) return 17;
-    return td == lstk::kTypeQ4_K ? 9 : td == lstk::kTypeQ8_0 ? 32 : 12;
+// 31 tokens. An all-Q4_K call of 64 tokens takes the path whatever its experts: fewer pairs were not measured slower there.
+bool grouped_pays(int tg, int td, long h, long f, int T, int k, int E) {
+    const bool q4 = tg == lstk::kTypeQ4_K && td == lstk::kTypeQ4_K, q8 = tg == lstk::kTypeQ8_0 || td == lstk::kTypeQ8_0;
+    const long weights = 3 * h * f, np = (long) T * k;
+    if (q4 && T >= 64) return true;
+    int from = 17;
+    if (weights < 1000000 || tg == lstk::kTypeQ8_0) from = 32;
+    else if (tg == lstk::kTypeQ4_K) from = q4 ? 9 : td == lstk::kTypeQ8_0 ? 32 : 12;
+    if (T < from || np < (q4 && weights >= 1000000 && weights < 2000000 ? 96 : 64)) return false;
+    return 4 * np >= (q4 ? 2 : q8 ? 6 : 3) * (long) E;
 }
 // LSTK_GROUPED_MIN_TOKENS, or -1 where it is not set.
 int grouped_env() {
@@ -874,7 +886,7 @@ int grouped_env() {
     return env ? std::max(1, std::atoi(env)) : -1;
 }
 bool takes_grouped(const lstk_moe_dims &d, int tu, int tg, int td, int n_slots, int T, int env) {
-    return T >= (env > 0 ? env : grouped_from(tg, td, d.n_embd, d.n_ff_exp)) &&
+    return (env > 0 ? T >= env : grouped_pays(tg, td, d.n_embd, d.n_ff_exp, T, d.n_expert_used, d.n_expert)) &&
            lstk::grouped_supported(tu, tg, td, d.n_embd, d.n_ff_exp, n_slots);
 }
 bool use_grouped(lstk_pool *P, const Shard &s, int T) {
@@ -892,16 +904,20 @@ bool use_grouped(lstk_pool *P, const Shard &s, int T) {
 // once: up to 4 pairs per expert on average most experts have one item, whose weights are read once: with the
 //   non-temporal hint they do not displace what is read again (us without / with: 64 evenly routed tokens of Q4_K 99 / 87,
 //   Q8_0 144 / 127, Q2_K + Q3_K 158 / 138; Zipf-routed, where hot experts' items share weights in L2, 58 / 61, 78 / 85,
-//   75 / 82; past 4 pairs that side loses more: 128 tokens of Q8_0 158 / 139 and 94 / 105).
+//   75 / 82; past 4 pairs that side loses more: 128 tokens of Q8_0 158 / 139 and 94 / 105). Q4_K past 64 tokens, where a hot
+//   expert may have more than four items and the staged kernels are close, only up to 2 pairs (256 experts, 8 used, f 512,
+//   Zipf-routed, staged kernels / without / with: 96 tokens 61 / 60 / 64, 128 68 / 66 / 71).
 struct GroupedPlan {
     bool rows;
     int chunk;
     bool once;
 };
-GroupedPlan grouped_plan(int tg, int td, int np, int n_expert) {
-    if (tg == lstk::kTypeQ4_K && td == lstk::kTypeQ4_K && np > 14 * n_expert) return {false, lstk::kGroupedChunk, false};
+GroupedPlan grouped_plan(int tg, int td, int T, int k, int n_expert) {
+    const int np = T * k;
+    const bool q4 = tg == lstk::kTypeQ4_K && td == lstk::kTypeQ4_K;
+    if (q4 && np > 14 * n_expert) return {false, lstk::kGroupedChunk, false};
     const bool q8 = tg == lstk::kTypeQ8_0 && td == lstk::kTypeQ8_0;
-    return {true, q8 && np > 12 * n_expert ? 32 : 16, np <= 4 * n_expert};
+    return {true, q8 && np > 12 * n_expert ? 32 : 16, np <= (q4 && T > 64 ? 2 : 4) * n_expert};
 }
 
 // The fused single-token path (one launch per block) is opt-in: LSTK_FUSED_DECODE=1 at pool creation.
@@ -1026,7 +1042,7 @@ int run_grouped(lstk_pool *P, const Shard &s, const CallScratch &sc, bool fixed,
     };
     const lstk_moe_dims &d = P->dims;
     const int k = d.n_expert_used, np = T * k, h = d.n_embd, f = d.n_ff_exp;
-    const auto [rows, chunk, once] = grouped_plan(s.tg, s.td, np, d.n_expert);
+    const auto [rows, chunk, once] = grouped_plan(s.tg, s.td, T, k, d.n_expert);
     const int max_items = lstk::grouped_max_items(np, (int) s.n_slots, chunk);
     const GroupedScratch &g = sc.grouped;
     lstk::PermuteParams pp{bins, np, (int) s.n_slots, chunk, g.counts, g.offsets, g.perm,
@@ -1482,7 +1498,7 @@ int lstk_debug_moe_plan(const lstk_moe_dims *dims, int type_gate, int type_down,
         dims->n_ff_exp < 256)
         return fail(LSTK_E_INVALID, "lstk_debug_moe_plan: bad arguments");
     const bool grouped = takes_grouped(*dims, type_gate, type_gate, type_down, n_slots, n_tokens, grouped_env());
-    const GroupedPlan g = grouped_plan(type_gate, type_down, n_tokens * dims->n_expert_used, dims->n_expert);
+    const GroupedPlan g = grouped_plan(type_gate, type_down, n_tokens, dims->n_expert_used, dims->n_expert);
     out[0] = grouped;
     out[1] = grouped && g.rows;
     out[2] = grouped ? g.chunk : 0;

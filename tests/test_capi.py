@@ -144,6 +144,36 @@ def test_noalloc_groups_only_in_its_own_scratch(lstk, types, h, f, E, k):
         lstk.moe_plan(types, h, f, E, k, 0)
 
 
+Q8, Q4, Q4KM, Q2XL = (8, 8, 8), (12, 12, 12), (12, 12, 14), (10, 10, 11)
+
+
+@pytest.mark.parametrize("h,f,E,k,first", [
+    (2048, 768, 128, 8, {Q8: 32, Q4: 9, Q4KM: 12, Q2XL: 17}),    # the shape the token counts were measured at
+    (2048, 768, 16, 2, {Q8: 32, Q4: 32, Q4KM: 32, Q2XL: 32}),    # 64 pairs (18 of Q4_K measured 27 us on the GEMV path, 34 grouped)
+    (2048, 768, 8, 1, {Q8: 64, Q4: 64, Q4KM: 64, Q2XL: 64}),
+    (1024, 512, 32, 4, {Q8: 32, Q4: 24, Q4KM: 16, Q2XL: 17}),    # 96 pairs for small Q4_K experts
+    (1024, 768, 128, 1, {Q8: 192, Q4: 64, Q4KM: 96, Q2XL: 96}),  # pairs per expert
+    (256, 512, 8, 2, {Q8: 32, Q4: 32, Q4KM: 32, Q2XL: 32}),
+])
+def test_grouped_path_starts_where_it_measured_no_slower(lstk, monkeypatch, h, f, E, k, first):
+    """The fewest tokens of a grouped call, and that every larger call is one too; the override counts tokens alone."""
+    for types, T0 in first.items():
+        assert [T for T in range(1, 513) if lstk.moe_plan(types, h, f, E, k, T)[0]] == list(range(T0, 513)), types
+    monkeypatch.setenv("LSTK_GROUPED_MIN_TOKENS", "5")
+    for types in first:
+        assert [lstk.moe_plan(types, h, f, E, k, T)[0] for T in (1, 4, 5, 6)] == [False, False, True, True]
+
+
+def test_kernels_of_a_grouped_call(lstk):
+    """Register-streaming or LDS-staged products, pairs per work item, non-temporal weights, by pairs per expert."""
+    plan = lambda t, T, E=128, k=8: lstk.moe_plan(t, 2048, 512, E, k, T)[1:4]
+    assert [plan(Q8, T) for T in (64, 65, 192, 193)] == [(True, 16, True), (True, 16, False), (True, 16, False), (True, 32, False)]
+    assert [plan(Q4, T) for T in (64, 65, 224, 225)] == [(True, 16, True), (True, 16, False), (True, 16, False), (False, 32, False)]
+    assert [plan(Q4, T, 256) for T in (64, 65, 448, 449)] == [(True, 16, True), (True, 16, False), (True, 16, False), (False, 32, False)]
+    assert [plan(Q2XL, T, 256) for T in (64, 128, 129)] == [(True, 16, True), (True, 16, True), (True, 16, False)]
+    assert [plan(Q4, T, 128, 2) for T in (64, 128, 129)] == [(True, 16, True), (True, 16, True), (True, 16, False)]
+
+
 def test_missing_library_fails_loudly(tmp_path, monkeypatch):
     import importlib
     import localstack_amd

@@ -32,12 +32,13 @@ def _ids(rng, T, reps):
     ((12, 12, 12), 256, 256, 64), ((12, 12, 12), 4096, 256, 64), ((10, 10, 11), 256, 512, 64), ((11, 11, 10), 512, 256, 63),
     ((13, 13, 14), 512, 256, 64), ((14, 14, 13), 256, 256, 33), ((12, 12, 14), 2048, 768, 64), ((12, 12, 8), 512, 256, 64),
     ((8, 8, 14), 256, 256, 320), ((10, 10, 11), 4096, 256, 64),
-    # up to 4 pairs per expert the weights are read with the non-temporal hint; each format at its fewest tokens
+    # up to 4 pairs per expert the weights are read with the non-temporal hint; few tokens
     ((8, 8, 8), 256, 256, 32), ((8, 8, 8), 4096, 256, 32), ((12, 12, 8), 512, 256, 32), ((12, 12, 12), 1024, 512, 9),
     ((12, 12, 14), 1024, 512, 12), ((10, 10, 11), 1024, 512, 17), ((11, 11, 10), 4096, 256, 17),
 ], ids=lambda v: "-".join(map(str, v)) if isinstance(v, tuple) else str(v))
-def test_rows_ffn_matches_oracle(orc, lstk, dev, types, h, f, T):
+def test_rows_ffn_matches_oracle(orc, lstk, dev, monkeypatch, types, h, f, T):
     import torch
+    monkeypatch.setenv("LSTK_GROUPED_MIN_TOKENS", "1")  # (16 experts: below 64 pairs the GEMV path is the default)
     E, k = 16, 2  # experts 8 .. 15 stay idle; 64 tokens take 16-pair items, more take 32 with Q8_0
     rng = np.random.default_rng(100 * types[0] + types[2] + h + f + T)
     up, gate, down = (synth.experts(rng, types[0], E, f, h, centered=True), synth.experts(rng, types[1], E, f, h, centered=True),
@@ -45,6 +46,7 @@ def test_rows_ffn_matches_oracle(orc, lstk, dev, types, h, f, T):
     x, resid = synth.activations(rng, T, h), synth.activations(rng, T, h)
     ids = _ids(rng, T, -(-T // 64))
     w = rng.uniform(0.1, 0.9, (T, k)).astype(np.float32)
+    assert lstk.moe_plan(types, h, f, E, k, T)[:2] == (True, True)
     store = lstk.ExpertStore(1, h, f, E, k, T, [(types, up, gate, down)])
     d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
     outs = []
