@@ -679,6 +679,13 @@ inline bool pick_split(int nsb, int *S, int *G) {
 // gate_up additionally needs 128 % G == 0 (rows per work-group = 128 / G).
 inline bool pick_split_gate_up(int nsb, int *S, int *G) { return pick_split(nsb, S, G) && 128 % *G == 0; }
 
+// Waits until at most N of the wavefront's vector memory operations are outstanding. A barrier alone does not promise that
+// global_load_lds copies have landed: a wavefront waits for its own before it meets the others, who read them.
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
 // Lets `kernel` take up to `bytes` of dynamic LDS (gfx950 has 160 KiB per CU; the default limit is 64) on the current
 // device. The limit is an attribute of a device's own copy of the kernel, so every device is asked once.
 inline hipError_t allow_dynamic_lds(const void *kernel, size_t bytes, std::atomic<uint64_t> &done) {

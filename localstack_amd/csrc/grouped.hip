@@ -231,10 +231,6 @@ __device__ __forceinline__ void dma16(const void *g, unsigned char *l) {
 __device__ __forceinline__ void dma4(const void *g, unsigned char *l) {
     __builtin_amdgcn_global_load_lds(g, (lds_void *) l, 4, 0, 0);
 }
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
 
 struct GLds {
     unsigned char *ring; // [kNS][kStageBytes]

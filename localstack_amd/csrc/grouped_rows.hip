@@ -504,6 +504,7 @@ __global__ __launch_bounds__(NW *kWave, WT == kTypeKQ8 ? (NW == 8 ? 2 : 3) : 4) 
         q[0].q[b] = load_q<WT, NT>(w0, b);
         q[1].q[b] = load_q<WT, NT>(w1, b);
     }
+    wait_vm<0>(); // this wavefront's copies into LDS (the weights, requested after them, are needed next anyway)
     __syncthreads();
     const int kg = lane / 16, r = lane % 16;
     f32x4 acc[2][MT];
