@@ -1,6 +1,6 @@
 """GPU parity of the many-token expert kernels that stream their weights through registers (grouped_rows.hip) against
-the oracle: every expert format, pair counts per expert at the edges of a 16- and a 32-pair work item (0, 1, 15, 16,
-17, 31, 32, 33), one and many super-blocks per row, and the two activation types in one layer.
+the oracle: every expert format, pair counts per expert at the edges of a 16- and a 32-pair work item (asserted, as is the
+kernel a call takes), one and many super-blocks per row, and the two activation types in one layer.
 
 Bar: the one of the other expert kernels (test_gpu_grouped.py): 2e-3 of the largest |out - resid|, for the f32 order
 over super-blocks, expf, and a SwiGLU value that rounds the other way into its 8 bits. Such a value moves an output by
@@ -27,24 +27,15 @@ def _ids(rng, T, reps):
     return np.stack(cols, 1)[:T].astype(np.int32)
 
 
-@pytest.mark.parametrize("types,h,f,T", [
-    ((8, 8, 8), 256, 256, 64), ((8, 8, 8), 256, 512, 320), ((8, 8, 8), 4096, 512, 64), ((8, 8, 8), 4096, 256, 64 * 3),
-    ((12, 12, 12), 256, 256, 64), ((12, 12, 12), 4096, 256, 64), ((10, 10, 11), 256, 512, 64), ((11, 11, 10), 512, 256, 63),
-    ((13, 13, 14), 512, 256, 64), ((14, 14, 13), 256, 256, 33), ((12, 12, 14), 2048, 768, 64), ((12, 12, 8), 512, 256, 64),
-    ((8, 8, 14), 256, 256, 320), ((10, 10, 11), 4096, 256, 64),
-    # up to 4 pairs per expert the weights are read with the non-temporal hint; few tokens
-    ((8, 8, 8), 256, 256, 32), ((8, 8, 8), 4096, 256, 32), ((12, 12, 8), 512, 256, 32), ((12, 12, 12), 1024, 512, 9),
-    ((12, 12, 14), 1024, 512, 12), ((10, 10, 11), 1024, 512, 17), ((11, 11, 10), 4096, 256, 17),
-], ids=lambda v: "-".join(map(str, v)) if isinstance(v, tuple) else str(v))
-def test_rows_ffn_matches_oracle(orc, lstk, dev, monkeypatch, types, h, f, T):
+def _ffn_against_oracle(orc, lstk, dev, types, h, f, T, ids, E=16, k=2):
+    """ids: int32 [T, k], or a function of the test's generator."""
     import torch
-    monkeypatch.setenv("LSTK_GROUPED_MIN_TOKENS", "1")  # (16 experts: below 64 pairs the GEMV path is the default)
-    E, k = 16, 2  # experts 8 .. 15 stay idle; 64 tokens take 16-pair items, more take 32 with Q8_0
     rng = np.random.default_rng(100 * types[0] + types[2] + h + f + T)
     up, gate, down = (synth.experts(rng, types[0], E, f, h, centered=True), synth.experts(rng, types[1], E, f, h, centered=True),
                       synth.experts(rng, types[2], E, h, f, centered=True))
     x, resid = synth.activations(rng, T, h), synth.activations(rng, T, h)
-    ids = _ids(rng, T, -(-T // 64))
+    if callable(ids):
+        ids = ids(rng)
     w = rng.uniform(0.1, 0.9, (T, k)).astype(np.float32)
     assert lstk.moe_plan(types, h, f, E, k, T)[:2] == (True, True)
     store = lstk.ExpertStore(1, h, f, E, k, T, [(types, up, gate, down)])
@@ -61,6 +52,40 @@ def test_rows_ffn_matches_oracle(orc, lstk, dev, monkeypatch, types, h, f, T):
     err = np.abs(outs[0] - ref).max() / np.abs(ref - resid).max()
     print(f"[rows {types} h={h} f={f} T={T}] rel max err {err:.3e}", flush=True)
     assert err <= FFN_TOL * max(1.0, (512 / f) ** 0.5)
+
+
+@pytest.mark.parametrize("types,h,f,T", [
+    ((8, 8, 8), 256, 256, 64), ((8, 8, 8), 256, 512, 320), ((8, 8, 8), 4096, 512, 64), ((8, 8, 8), 4096, 256, 64 * 3),
+    ((12, 12, 12), 256, 256, 64), ((12, 12, 12), 4096, 256, 64), ((10, 10, 11), 256, 512, 64), ((11, 11, 10), 512, 256, 63),
+    ((13, 13, 14), 512, 256, 64), ((14, 14, 13), 256, 256, 33), ((12, 12, 14), 2048, 768, 64), ((12, 12, 8), 512, 256, 64),
+    ((8, 8, 14), 256, 256, 320), ((10, 10, 11), 4096, 256, 64),
+    # up to 4 pairs per expert the weights are read with the non-temporal hint; few tokens
+    ((8, 8, 8), 256, 256, 32), ((8, 8, 8), 4096, 256, 32), ((12, 12, 8), 512, 256, 32), ((12, 12, 12), 1024, 512, 9),
+    ((12, 12, 14), 1024, 512, 12), ((10, 10, 11), 1024, 512, 17), ((11, 11, 10), 4096, 256, 17),
+], ids=lambda v: "-".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_rows_ffn_matches_oracle(orc, lstk, dev, monkeypatch, types, h, f, T):
+    monkeypatch.setenv("LSTK_GROUPED_MIN_TOKENS", "1")  # (16 experts: below 64 pairs the GEMV path is the default)
+    # experts 8 .. 15 stay idle; 64 tokens take 16-pair items, more take 32 with Q8_0
+    _ffn_against_oracle(orc, lstk, dev, types, h, f, T, lambda rng: _ids(rng, T, -(-T // 64)))
+
+
+# pairs per expert, every count a remainder of its item size or a whole number of items
+@pytest.mark.parametrize("types,chunk,counts", [
+    # 32-pair items need more than 12 pairs per expert on average over the pool's 8
+    ((8, 8, 8), 32, (1, 31, 32, 33, 17, 16, 15, 47)), ((8, 8, 8), 32, (64, 63, 48, 49, 30, 0, 2, 18)),
+    ((8, 8, 8), 16, (1, 15, 16, 17, 31, 0, 2, 14)), ((12, 12, 12), 16, (1, 15, 16, 17, 31, 32, 0, 0)),
+    ((10, 10, 11), 16, (1, 15, 16, 17, 31, 32, 33, 47)), ((12, 12, 14), 16, (63, 33, 31, 17, 16, 15, 1, 0)),
+], ids=lambda v: "-".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_pair_counts_at_the_edges_of_an_item(orc, lstk, dev, monkeypatch, types, chunk, counts):
+    monkeypatch.setenv("LSTK_GROUPED_MIN_TOKENS", "1")
+    rng, n = np.random.default_rng(sum(types) + chunk), sum(counts)
+    assert n % 2 == 0
+    # two columns: the sorted list's halves hold no expert at the same place unless it has more than half of all pairs
+    flat = np.repeat(np.arange(8), counts)
+    ids = np.stack([flat[:n // 2], flat[n // 2:]], 1)[rng.permutation(n // 2)].astype(np.int32)
+    assert (ids[:, 0] != ids[:, 1]).all() and tuple(np.bincount(ids.ravel(), minlength=8)) == counts
+    assert lstk.moe_plan(types, 512, 512, 8, 2, n // 2)[:3] == (True, True, chunk)
+    _ffn_against_oracle(orc, lstk, dev, types, 512, 512, n // 2, ids, E=8)
 
 
 @pytest.mark.parametrize("wtype", (8, 12))
