@@ -1270,6 +1270,7 @@ struct AttnSplitLds {
     uint16_t list[kAsMapBlocks]; // the live blocks in order
     int n_live;
 };
+static_assert(sizeof(AttnSplitLds<128>) <= 160 * 1024, "a CU's LDS");
 
 template <int HD>
 __global__ __launch_bounds__(kAsWaves *kWave) void attn_split_kernel(AttnParams P) {

@@ -1,6 +1,6 @@
 """CPU replay of the attention launch plan and of every index the attention kernels compute
-(localstack_amd/csrc/forward.hip: attn_plan, attn_kernel, attn1_kernel, attn_rows_kernel, attn_combine_kernel; buffers sized as
-model.cpp allocates them), for work-group targets of 512 (the build's; halved for steps of a few tokens in
+(localstack_amd/csrc/forward.hip: attn_plan, attn_kernel, attn1_kernel, attn_rows_kernel, attn_split_kernel, attn_combine_kernel;
+buffers sized as model.cpp allocates them), for work-group targets of 512 (the build's; halved for steps of a few tokens in
 one row block), 256 and 128, over the shapes the
 tests and the benchmark run and past them: every global index stays inside its buffer, every LDS index
 inside its array, and the partial rows inside attn_part_rows. No GPU. The replayed plan is held equal to
@@ -19,6 +19,7 @@ AT_BLOCK = 256      # kAtBlock: 4 wavefronts
 MAX_PASSES = 2048   # kAttnMaxPasses: passes per chunk the skip map of many-token steps covers
 BLOCK = 256         # kBlock (attn_combine_kernel)
 LDS_MAX = 65536
+LDS_CU = 160 * 1024 # of a CU; attn_split_kernel asks for it (allow_dynamic_lds)
 A1_WGS = 256        # kAttn1Wgs: one work-group per CU
 
 
@@ -125,6 +126,8 @@ def check_launch(T, n_head, n_kv, hd, kv_size, n_cells, n_batch, target, rope_in
         assert (cv % 4 == 0).all() and cv.min() >= 0 and cv.max() + 3 < kv_size
         lds = 16 * 128 * 4 + 2 * 128 * 2 + NW * 16 * 132 * 4 + 2 * NW * 16 * 4
         assert lds == {4: 43008, 5: 51584, 6: 60160}[NW] and lds <= LDS_MAX  # the compiler's figures
+    elif split(T, n_head, n_kv, n_cells, target, cell_begin, hd):
+        check_split(n_kv, hd, kv_size, begin, end, chunk, kv_elems)
     elif rb_rows == 64 and hd <= 128:
         # attn_rows_kernel: wavefront w fetches K of cell b0 + 16 w + lr, V of cells b0 + 16 w + 4 lq ..
         # + 3 and the cell tables of cell b0 + 16 w + (lane & 15), clamped to the cache; partial rows and
@@ -150,7 +153,7 @@ def check_launch(T, n_head, n_kv, hd, kv_size, n_cells, n_batch, target, rope_in
         lds = (RB * FA_CELLS * 4 + 2 * RB * (FA_CELLS + 8) * 2 + 3 * RB * 4 + RB * 4 + (16 * hd if NRT == 1 else 1) * 4 +
                (MAX_PASSES if skip else 1))
         assert lds <= LDS_MAX
-    if skip:  # the skip map holds one byte per pass of the chunk
+    if skip and not split(T, n_head, n_kv, n_cells, target, cell_begin, hd):  # the skip map holds one byte per pass of the chunk
         assert (chunk + FA_CELLS - 1) // FA_CELLS <= MAX_PASSES
     # outputs: n_chunk == 1 writes out[(t * n_head + h) * hd + d]; else part rows
     if n_chunk > 1:
@@ -164,6 +167,40 @@ def check_launch(T, n_head, n_kv, hd, kv_size, n_cells, n_batch, target, rope_in
         assert clds <= LDS_MAX
         assert ((T - 1) * n_head + n_head - 1) * n_chunk + n_chunk - 1 < part_rows(n_batch, n_head)
     return rb_rows, n_rowblk, chunk, n_chunk, rope_in
+
+
+def check_split(n_kv, hd, kv_size, begin, end, chunk, kv_elems):
+    """attn_split_kernel<hd> over chunks [begin, end): 8 wavefronts, 16-cell units, byte offsets of 32 bits per lane above a
+    head's base; a block map of 2 MAX_PASSES entries where the chunk's passes fit it."""
+    NK = hd // 16
+    # LDS: {at [4096] u16 or o [8][4][NK / 2][64] float4}, q [4][NK / 2][64] 16 B, m / l [8][64] f32, list [4096] u16, n_live
+    lds = max(2 * 2 * MAX_PASSES, 8 * 4 * (NK // 2) * 64 * 16) + 4 * (NK // 2) * 64 * 16 + 2 * 8 * 64 * 4 + 2 * 2 * MAX_PASSES + 4
+    lds = (lds + 15) // 16 * 16
+    assert lds == {64: 86032, 128: 159760}[hd] and lds <= LDS_CU  # sizeof(AttnSplitLds<hd>)
+    lq, lr = np.arange(4)[:, None], np.arange(16)[None, :]
+    for b0, e0 in zip(begin, end):
+        n_pass = -(-(e0 - b0) // FA_CELLS)
+        skip = n_pass <= MAX_PASSES
+        assert b0 % 32 == 0 and (not skip or 2 * n_pass <= 2 * MAX_PASSES <= 0xffff)  # lane 0 / 32 at a block's first cell; entries u16
+        # the map: a pass's 64 cells (table entries clamped to the cache), positions below 32 * 4096 where the order is by position
+        assert np.minimum(b0 + 64 * n_pass - 1, kv_size - 1) < kv_size
+        if kv_size <= 32 * 2 * MAX_PASSES:
+            assert (kv_size - 1) // 32 < 2 * MAX_PASSES  # a position never exceeds the cells of the cache
+        # units: both halves of every block a pass can hold, or every 16 cells; the extremes of the chunk bound the rest
+        units = np.unique(np.array([b0, b0 + 16, b0 + (e0 - b0) // 2 // 16 * 16, b0 + 64 * n_pass - 32, b0 + 64 * n_pass - 16]))
+        for u in units:
+            cc = np.minimum(u + lr, kv_size - 1)
+            k_off = (lq * kv_size + cc) * 8
+            k_top = (n_kv - 1) * hd * kv_size * 2 + (NK - 1) * 32 * kv_size + k_off.max() + 8
+            v_cell = np.minimum(u + 4 * lq, kv_size - 4)
+            assert (v_cell % 4 == 0).all() and v_cell.min() >= 0
+            v_off = (v_cell // 4 * hd + lr) * 8
+            v_top = (n_kv - 1) * hd * kv_size * 2 + 128 * (NK - 1) + v_off.max() + 8
+            assert max(k_off.max(), v_off.max()) < 1 << 32 and max(k_top, v_top) <= 2 * kv_elems
+    # the merge: wavefront w finishes tile w / 2 and NO dim tiles of each half; every (tile, dim tile) once
+    NH, NO = NK // 2, NK // 4
+    done = [(w >> 1, half * NH + (w & 1) * NO + d) for w in range(8) for half in range(2) for d in range(NO)]
+    assert sorted(done) == [(rt, dt) for rt in range(4) for dt in range(NK)]
 
 
 def test_replayed_plan_is_the_library_plan(lstk):
@@ -226,6 +263,19 @@ def check_cells(n_head, n_kv, hd, grp, n_cells, kv_size, target):
                              cell_begin=(n_cells - 256) // 64 * 64)
                 plans += 1
     return plans
+
+
+@pytest.mark.parametrize("heads,hd", [((48, 16), 128), ((80, 16), 64), ((8, 8), 128), ((128, 32), 64)], ids=str)
+def test_split_indices_of_other_query_groups(heads, hd):
+    """Groups of 3, 5, 1 and 4 query heads, row blocks that end inside a tile, a cache past the order by position and a chunk
+    past the block map."""
+    n = 0
+    for T in (64, 65, 127, 200, 256, 341, 512):
+        for kv_size, cells in ((2048, 512), (2048, 1280), (8192, 8192), (65536, 65536), (132096, 131328), (132096, 1280)):
+            if split(T, *heads, cells, hd=hd):
+                check_launch(T, *heads, hd, kv_size, cells, 512, 512, False)
+                n += 1
+    assert n >= 15, n
 
 
 def test_rope_in_keeps_single_pass_chunks():
