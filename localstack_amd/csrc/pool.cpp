@@ -223,23 +223,23 @@ size_t grouped_scratch(const lstk_moe_dims &d, int T, int n_bins, uint8_t *base,
     auto take = [&](size_t bytes) {
         const size_t o = off;
         off = align_up(off + bytes, 256);
-        return base + o;
+        return o;
     };
-    uint8_t *counts = take(nb * 4), *offsets = take((nb + 1) * 4), *perm = take(np * 4), *n_items = take(64);
-    uint8_t *items = take((size_t) lstk::grouped_max_items((int) np, n_bins, 16) * 16); // 16: the shortest work items
-    uint8_t *qs = take(np * f), *ad = take(np * (f / 32) * 4), *bs = take(np * (f / 32) * 4), *bh = take(np * (f / 32) * 4);
-    uint8_t *xbh = take(t * (h / 32) * 4);
+    const size_t counts = take(nb * 4), offsets = take((nb + 1) * 4), perm = take(np * 4), n_items = take(64);
+    const size_t items = take((size_t) lstk::grouped_max_items((int) np, n_bins, 16) * 16); // 16: the shortest work items
+    const size_t qs = take(np * f), ad = take(np * (f / 32) * 4), bs = take(np * (f / 32) * 4), bh = take(np * (f / 32) * 4);
+    const size_t xbh = take(t * (h / 32) * 4);
     if (base && out) {
-        out->counts = reinterpret_cast<int32_t *>(counts);
-        out->offsets = reinterpret_cast<int32_t *>(offsets);
-        out->perm = reinterpret_cast<int32_t *>(perm);
-        out->n_items = reinterpret_cast<int32_t *>(n_items);
-        out->items = reinterpret_cast<int4 *>(items);
-        out->aq.qs = reinterpret_cast<int8_t *>(qs);
-        out->aq.d = reinterpret_cast<float *>(ad);
-        out->aq.bs = reinterpret_cast<int32_t *>(bs);
-        out->aq.bh = reinterpret_cast<uint32_t *>(bh);
-        out->xbh = reinterpret_cast<uint32_t *>(xbh);
+        out->counts = reinterpret_cast<int32_t *>(base + counts);
+        out->offsets = reinterpret_cast<int32_t *>(base + offsets);
+        out->perm = reinterpret_cast<int32_t *>(base + perm);
+        out->n_items = reinterpret_cast<int32_t *>(base + n_items);
+        out->items = reinterpret_cast<int4 *>(base + items);
+        out->aq.qs = reinterpret_cast<int8_t *>(base + qs);
+        out->aq.d = reinterpret_cast<float *>(base + ad);
+        out->aq.bs = reinterpret_cast<int32_t *>(base + bs);
+        out->aq.bh = reinterpret_cast<uint32_t *>(base + bh);
+        out->xbh = reinterpret_cast<uint32_t *>(base + xbh);
     }
     return off;
 }
@@ -1002,18 +1002,18 @@ size_t call_scratch_layout(const lstk_moe_dims &d, int T, uint8_t *base, CallScr
     auto take = [&](size_t bytes) {
         const size_t o = off;
         off = align_up(off + bytes, 256);
-        return base + o;
+        return o;
     };
-    uint8_t *qs = take(t * h), *xd = take(t * (h / 32) * 4), *bs = take(t * (h / 32) * 4);
-    uint8_t *lg = take(t * (size_t) d.n_expert * 4), *act = take(t * k * (size_t) d.n_ff_exp * 4), *Y = take(t * k * h * 4);
+    const size_t qs = take(t * h), xd = take(t * (h / 32) * 4), bs = take(t * (h / 32) * 4);
+    const size_t lg = take(t * (size_t) d.n_expert * 4), act = take(t * k * (size_t) d.n_ff_exp * 4), Y = take(t * k * h * 4);
     if (base && out) {
-        out->xq.qs = reinterpret_cast<int8_t *>(qs);
-        out->xq.d = reinterpret_cast<float *>(xd);
-        out->xq.bs = reinterpret_cast<int32_t *>(bs);
+        out->xq.qs = reinterpret_cast<int8_t *>(base + qs);
+        out->xq.d = reinterpret_cast<float *>(base + xd);
+        out->xq.bs = reinterpret_cast<int32_t *>(base + bs);
         out->xq.bh = nullptr;
-        out->logits = reinterpret_cast<float *>(lg);
-        out->act = reinterpret_cast<float *>(act);
-        out->Y = reinterpret_cast<float *>(Y);
+        out->logits = reinterpret_cast<float *>(base + lg);
+        out->act = reinterpret_cast<float *>(base + act);
+        out->Y = reinterpret_cast<float *>(base + Y);
     }
     return off;
 }
