@@ -17,7 +17,9 @@ only to own device memory and streams. There is no CPU fallback: every compute c
 kernels, and a missing library raises.
 """
 import ctypes
+import gc
 import os
+import weakref
 
 import numpy as np
 
@@ -247,6 +249,9 @@ def unpack_matrix(type_, rows, cols, packed):
     return out
 
 
+_stores = weakref.WeakSet()  # stores not yet freed
+
+
 class ExpertStore:
     """The HBM expert pool (ExpertStore, src/expert_store.h:113-131) and the MoE calls that read it.
 
@@ -269,6 +274,11 @@ class ExpertStore:
                     self._keep.append(a)
                     ptrs.append(a.ctypes.data)
             arr[l] = ExpertLayer(types[0], types[1], types[2], *ptrs)
+        # A store dropped in a reference cycle, and the graphs that replay it, stay until Python's cyclic collector runs. Their
+        # HBM is wanted now; and a collection that falls into a later stream capture would free device memory and destroy
+        # graphs there, which HIP refuses (torch ends the process). 65 ms beside torch, and only where another store is left.
+        if not dry and _stores:
+            gc.collect()
         flags = ((POOL_STREAMING if streaming else 0) | (POOL_DRY if dry else 0) | (POOL_DEVICE_LRU if device_lru else 0) |
                  (POOL_AUTO_SIZE if auto_size else 0))
         h = ctypes.c_void_p()
@@ -277,6 +287,7 @@ class ExpertStore:
         self._h = h
         self._keep = None  # the pool copied what it needs
         self._destroy = lib().lstk_pool_destroy  # held, so that closing works during interpreter shutdown
+        _stores.add(self)
 
     def close(self):
         if getattr(self, "_h", None):

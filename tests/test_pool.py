@@ -207,3 +207,32 @@ def test_auto_size_needs_a_device_pool(lstk):
     with pytest.raises(lstk.LstkError, match="AUTO_SIZE"):
         lstk.ExpertStore(2, 256, 512, 8, 2, 4, [((8,) * 3, None, None, None)] * 2, pool_bytes=0, min_slots=8,
                          streaming=True, dry=True, auto_size=True)
+
+
+def test_a_new_store_frees_the_ones_dropped_in_cycles(lstk):
+    """A store held by a reference cycle (a state dict whose step function holds the dict) is freed, with whatever else the
+    cycle holds, before another one is created, not at some later allocation (a stream capture may be running then)."""
+    import functools
+    import gc
+    import weakref
+
+    class Graph:
+        pass
+
+    def state():
+        st = {"store": lstk.ExpertStore(1, 256, 512, 8, 2, 4, [((8, 8, 8), None, None, None)], dry=True), "graph": Graph()}
+        st["step"] = functools.partial(len, st)
+        return weakref.ref(st["graph"]), weakref.ref(st["store"])
+
+    gc.disable()
+    try:
+        refs = state()
+        assert all(r() is not None for r in refs)
+        lstk.ExpertStore(1, 256, 512, 8, 2, 4, [((8, 8, 8), None, None, None)], dry=True).close()
+        assert all(r() is not None for r in refs)  # a dry store holds no HBM and is not captured
+        # null tensors: refused by a device and without one, after the collection
+        with pytest.raises(lstk.LstkError):
+            lstk.ExpertStore(1, 256, 512, 8, 2, 4, [((8, 8, 8), None, None, None)])
+        assert all(r() is None for r in refs)
+    finally:
+        gc.enable()
