@@ -24,9 +24,10 @@
 // Integer sums are those of ggml's vec_dot; only the f32 order over super-blocks differs.
 //
 // Bound: the expert bytes while an expert has a few pairs (64 tokens through a 30B-shaped Q2_K + Q3_K layer: 153 us for
-// 717 MB of unpacked weights), VALU work on the products past that. Against the GEMV kernels, which served these calls
+// 717 MB of unpacked weights); past that the bytes of an expert's items, fetched about once (1.05 to 1.11 times the weights) at 3.5
+// to 4.3 TB/s, beside VALU work that keeps the VALU half busy (512 Q8_0 tokens 51% and 45%, matrix cores 15% and 12%). Against the GEMV kernels, which served these calls
 // before with dot products on the VALU and a work-group per expert however many pairs it had, on 30B-shaped layers on
-// MI355X: 512 tokens Q8_0 630 -> 200 us a layer, 203 tokens Q4_K + Q6_K 329 -> 132, 64 tokens Q2_K + Q3_K 200 -> 153 (-> 134 with
+// MI355X: 512 tokens Q8_0 630 -> 202 us a layer, 203 tokens Q4_K + Q6_K 329 -> 130, 64 tokens Q2_K + Q3_K 200 -> 153 (-> 134 with
 // the weights' non-temporal loads of calls whose experts mostly have one item, GroupedParams::once).
 #include "device.h"
 #include "formats.h"
@@ -546,7 +547,8 @@ hipError_t launch_rows_n(const GroupedParams &P, int max_items, hipStream_t st, 
 // work-groups a CU holds then are 16 wavefronts: 30B-shaped Q8_0 layer, 32-pair items, us with 4 / 8: 300 Zipf-routed
 // tokens 145 / 129, 512 194 / 181, 512 evenly routed 218 / 220; 235B shape, 16-pair Q4_K items, 64 tokens 315 / 295.
 // Below that 4 are faster (more work-groups overlap their starts: 64 tokens of Q2_K + Q3_K 159 / 186), and so they are
-// for down, whose rows are short (512 tokens Q8_0 214 / 244).
+// for down, whose rows are short (512 tokens Q8_0 214 / 244). (Q8_0 figures from before the super-block sums, which add 1 to 2%
+// to either side.)
 template <int WT, bool MINS, int MT, bool DOWN, bool NT>
 hipError_t launch_rows_w(const GroupedParams &P, int max_items, hipStream_t st, const LaunchTiming *tm) {
     if constexpr (!DOWN)

@@ -899,7 +899,7 @@ bool use_grouped(lstk_pool *P, const Shard &s, int T) {
 //   kernels of grouped.hip against rows, us: 64 tokens 106 / 98, 128 115 / 103, 203 122 / 113, 256 123 / 126, 512 166 / 180;
 //   the staged kernels build their weight planes once per 32 pairs and win when the pairs fill them).
 // chunk: 16 pairs (one matrix-core tile, 36 KB of LDS at h 2048) or, for Q8_0 past 12 pairs per expert, 32 (us: 200
-//   tokens 165 / 165, 256 181 / 174, 400 214 / 199, 300 Zipf-routed 153 / 137). KQ8 stays at 16: its second tile takes
+//   tokens 165 / 165, 256 181 / 174, 400 214 / 199, 300 Zipf-routed 153 / 137, from before the super-block sums). KQ8 stays at 16: its second tile takes
 //   the kernel past 200 VGPRs (203 tokens 135 / 200).
 // once: up to 4 pairs per expert on average most experts have one item, whose weights are read once: with the
 //   non-temporal hint they do not displace what is read again (us without / with: 64 evenly routed tokens of Q4_K 99 / 87,
