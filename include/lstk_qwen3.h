@@ -148,9 +148,9 @@ int lstk_model_debug_options(lstk_model *model, int flags);
 int lstk_debug_attn_plan(int n_tokens, int n_head, int n_kv, int head_dim, int kv_size, int n_cells, int cell_begin,
                          int rope_in, int32_t out[6]);
 /* Test hook: whether such a step's attention (no RoPE inside) splits the cells over a work-group's wavefronts (1) or the
- * query rows (0). */
+ * query rows (0); n_live = cells of the range that belong to the sequence (0: all). */
 int lstk_debug_attn_split(int n_tokens, int n_head, int n_kv, int head_dim, int kv_size, int n_cells, int cell_begin,
-                          int32_t *split);
+                          int n_live, int32_t *split);
 
 /* Engine::set_routing_trace (src/engine.cpp:179-186): with a path, creates the file and writes the
  * trace header ("LSTKRTE1", n_layer, n_expert, n_expert_used as little-endian int32); every later step

@@ -133,7 +133,7 @@ SIGNATURES = {
     "lstk_dequant_f16": (_I, [_I, _P, ctypes.c_size_t, _P]),
     "lstk_model_set_timing": (_I, [_P, _I]),
     "lstk_debug_attn_plan": (_I, [_I, _I, _I, _I, _I, _I, _I, _I, _P]),
-    "lstk_debug_attn_split": (_I, [_I, _I, _I, _I, _I, _I, _I, ctypes.POINTER(ctypes.c_int32)]),
+    "lstk_debug_attn_split": (_I, [_I, _I, _I, _I, _I, _I, _I, _I, ctypes.POINTER(ctypes.c_int32)]),
     "lstk_debug_moe_plan": (_I, [ctypes.POINTER(MoeDims), _I, _I, _I, _I, _P]),
     "lstk_model_debug_options": (_I, [_P, _I]),
     "lstk_model_timing": (_I, [_P, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_int64)]),
@@ -217,11 +217,12 @@ def attn_plan(n_tokens, n_head, n_kv, head_dim, kv_size, n_cells, cell_begin=0, 
     return out[0], out[1], out[2], out[3], bool(out[4]), out[5]
 
 
-def attn_split(n_tokens, n_head, n_kv, head_dim, kv_size, n_cells, cell_begin=0):
-    """Whether a step's attention splits the cells over a work-group's wavefronts (host arithmetic, no device call)."""
+def attn_split(n_tokens, n_head, n_kv, head_dim, kv_size, n_cells, cell_begin=0, n_live=0):
+    """Whether a step's attention splits the cells over a work-group's wavefronts (host arithmetic, no device call); n_live =
+    cells of the range that belong to the sequence (0: all)."""
     out = ctypes.c_int32()
     _check(lib().lstk_debug_attn_split(int(n_tokens), int(n_head), int(n_kv), int(head_dim), int(kv_size), int(n_cells),
-                                       int(cell_begin), ctypes.byref(out)))
+                                       int(cell_begin), int(n_live), ctypes.byref(out)))
     return bool(out.value)
 
 

@@ -564,6 +564,7 @@ int forward(lstk_model *M, int32_t seq, int T, int n_cells, float *d_logits, int
         ap.kv_size = (int) M->kv.size;
         ap.n_cells = n_cells;
         ap.cell_begin = range_begin;
+        ap.n_live = M->kv.length(seq);
         ap.scale = 1.0f / sqrtf((float) hd);
         ap.part = M->part;
         ap.out = M->attn;
@@ -811,7 +812,7 @@ int lstk_model_debug_options(lstk_model *model, int flags) {
 }
 
 static int planned(int n_tokens, int n_head, int n_kv, int head_dim, int kv_size, int n_cells, int cell_begin, int rope_in,
-                   lstk::AttnParams &ap) {
+                   int n_live, lstk::AttnParams &ap) {
     if (n_tokens < 1 || n_head < 1 || n_kv < 1 || n_head % n_kv || !lstk::attn_supported(head_dim) || kv_size < 32 ||
         kv_size % 32 || n_cells < 1 || n_cells > kv_size || cell_begin < 0 || cell_begin >= n_cells || cell_begin % 64)
         return set_error(LSTK_E_INVALID, "attention plan: bad arguments");
@@ -823,6 +824,7 @@ static int planned(int n_tokens, int n_head, int n_kv, int head_dim, int kv_size
     ap.n_cells = n_cells;
     ap.cell_begin = cell_begin;
     ap.rope_in = rope_in ? 1 : 0;
+    ap.n_live = n_live;
     lstk::attn_plan(ap);
     return LSTK_OK;
 }
@@ -831,7 +833,7 @@ int lstk_debug_attn_plan(int n_tokens, int n_head, int n_kv, int head_dim, int k
                          int rope_in, int32_t out[6]) {
     if (!out) return set_error(LSTK_E_INVALID, "null argument");
     lstk::AttnParams ap{};
-    const int rc = planned(n_tokens, n_head, n_kv, head_dim, kv_size, n_cells, cell_begin, rope_in, ap);
+    const int rc = planned(n_tokens, n_head, n_kv, head_dim, kv_size, n_cells, cell_begin, rope_in, 0, ap);
     if (rc != LSTK_OK) return rc;
     out[0] = ap.rb_rows;
     out[1] = ap.n_rowblk;
@@ -843,10 +845,10 @@ int lstk_debug_attn_plan(int n_tokens, int n_head, int n_kv, int head_dim, int k
 }
 
 int lstk_debug_attn_split(int n_tokens, int n_head, int n_kv, int head_dim, int kv_size, int n_cells, int cell_begin,
-                          int32_t *split) {
+                          int n_live, int32_t *split) {
     if (!split) return set_error(LSTK_E_INVALID, "null argument");
     lstk::AttnParams ap{};
-    const int rc = planned(n_tokens, n_head, n_kv, head_dim, kv_size, n_cells, cell_begin, 0, ap);
+    const int rc = planned(n_tokens, n_head, n_kv, head_dim, kv_size, n_cells, cell_begin, 0, n_live, ap);
     if (rc != LSTK_OK) return rc;
     *split = lstk::attn_in_split(ap) ? 1 : 0;
     return LSTK_OK;

@@ -53,12 +53,15 @@ def plan(T, n_head, n_kv, n_cells, target=512, rope_in=False, cell_begin=0, hd=1
     return rb_rows, n_rowblk, chunk, n_chunk, rope_in
 
 
-def split(T, n_head, n_kv, n_cells, target=512, cell_begin=0, hd=128):
+def split(T, n_head, n_kv, n_cells, target=512, cell_begin=0, hd=128, n_live=0):
     """attn_in_split (forward.hip): whether a planned launch without RoPE splits the cells over its wavefronts."""
     rb_rows, n_rowblk, chunk, n_chunk, _ = plan(T, n_head, n_kv, n_cells, target, False, cell_begin, hd)
     if T < 64 or rb_rows != 64 or hd > 128:
         return False
-    return chunk >= (192 if n_kv * n_rowblk * n_chunk <= A1_WGS else 768 if hd == 64 else 576)
+    one_round = n_kv * n_rowblk * n_chunk <= A1_WGS
+    if 0 < n_live < (192 if one_round else 256):
+        return False
+    return chunk >= (192 if one_round else 768 if hd == 64 else 576)
 
 
 def part_rows(n_batch, n_head):
@@ -220,8 +223,9 @@ def test_replayed_plan_is_the_library_plan(lstk):
                             assert got[5] == n_kv * want[1] * want[3]
                             cases += 1
                         if T > 1:
-                            assert lstk.attn_split(T, n_head, n_kv, hd, kv_size, n_cells, cell_begin) == \
-                                split(T, n_head, n_kv, n_cells, 512, cell_begin, hd), (n_head, n_cells, cell_begin, T)
+                            for live in (0, 191, 192, 255, 256):
+                                assert lstk.attn_split(T, n_head, n_kv, hd, kv_size, n_cells, cell_begin, live) == \
+                                    split(T, n_head, n_kv, n_cells, 512, cell_begin, hd, live), (n_head, n_cells, cell_begin, T)
     assert cases > 1000
     with pytest.raises(lstk.LstkError):
         lstk.attn_plan(1, 32, 4, 128, 1000, 256)  # kv_size not a multiple of 32
@@ -305,6 +309,8 @@ def test_short_chunks_keep_the_row_split(lstk):
     assert not any(ask(T, 2048) for T in (64, 96, 128)) and ask(384, 2048) and ask(256, 4000) and ask(64, 16000)
     assert not any(ask(T, c, (4, 2), 64) for T in (64, 256, 512) for c in (0, 512, 2048)) and ask(512, 16000, (4, 2), 64)
     assert not ask(512, 4000, (16, 2), 256)  # head size 256 has no such kernel
+    # a short sequence whose blocks lie far apart: long chunks, but few live cells in them
+    assert [lstk.attn_split(128, 32, 4, 128, 65536, 32768, 0, n) for n in (192, 255, 256, 0)] == [False, False, True, True]
     with pytest.raises(lstk.LstkError):
         lstk.attn_split(64, 32, 4, 128, 1000, 256)
 

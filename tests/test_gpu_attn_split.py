@@ -108,7 +108,7 @@ def _compare(got, ref, what):
 
 
 # heads, head size, tokens, context, cache cells, (cells per chunk, chunks) in the plain layout
-LONG = [((128, 32), 64, 113, 0, 2048, (256, 1)), ((128, 32), 64, 128, 900, 2048, (1280, 1)), ((80, 16), 64, 193, 523, 2048, (768, 1)),
+LONG = [((128, 32), 64, 113, 100, 2048, (256, 1)), ((128, 32), 64, 128, 900, 2048, (1280, 1)), ((80, 16), 64, 193, 523, 2048, (768, 1)),
         ((80, 16), 64, 204, 60, 2048, (512, 1)), ((128, 32), 64, 70, 3300, 4096, (896, 4)),
         ((48, 16), 128, 321, 900, 2048, (1280, 1)), ((48, 16), 128, 341, 3, 2048, (512, 1)), ((64, 8), 128, 250, 0, 2048, (256, 1)),
         ((64, 8), 128, 255, 600, 2048, (1024, 1)), ((48, 16), 128, 200, 2300, 4096, (640, 4)), ((8, 8), 128, 64, 6000, 8192, (192, 32)),
@@ -121,7 +121,7 @@ def test_long_chunks_match_64_bits(lstk, dev, heads, hd, T, ctx, kv_size, want):
     chunk, whose sums are taken in the order of the positions)."""
     hp, w = _one_layer(*heads, hd)
     cells = (ctx + T + 255) // 256 * 256
-    assert lstk.attn_plan(T, *heads, hd, kv_size, cells)[2:4] == want and lstk.attn_split(T, *heads, hd, kv_size, cells)
+    assert lstk.attn_plan(T, *heads, hd, kv_size, cells)[2:4] == want and lstk.attn_split(T, *heads, hd, kv_size, cells, 0, ctx + T)
     toks, pos = prompt(T + ctx, T, hp["n_vocab"]), np.arange(ctx, ctx + T)
     q, k, v = _qkv(hp, w, toks, pos)
     kc, vc = (a.astype(np.float64).reshape(ctx, heads[1], hd) for a in synthetic_kv(9, 0, 0, ctx, heads[1], hd))
@@ -146,19 +146,19 @@ def test_long_chunks_match_64_bits(lstk, dev, heads, hd, T, ctx, kv_size, want):
 
 
 def test_block_whose_first_cells_were_never_written(lstk, dev):
-    """32 tokens, then 5 cells reserved by a prepare whose forward never ran, then a 120-token step: the second block's first
-    cells hold no position, and the step sees its other cells and the first block."""
-    heads, hd, T = (128, 32), 64, 120
+    """96 tokens, then 5 cells reserved by a prepare whose forward never ran, then a 120-token step: the fourth block's first
+    cells hold no position, and the step sees its other cells and the blocks before it."""
+    heads, hd, T, n = (128, 32), 64, 120, 96
     hp, w = _one_layer(*heads, hd)
-    assert lstk.attn_split(T, *heads, hd, 512, 256)
-    toks = prompt(3, 32 + T, hp["n_vocab"])
-    pos = np.concatenate([np.arange(32), 37 + np.arange(T)])
+    assert lstk.attn_split(T, *heads, hd, 512, 256, 0, n + 5 + T)
+    toks = prompt(3, n + T, hp["n_vocab"])
+    pos = np.concatenate([np.arange(n), n + 5 + np.arange(T)])
     q, k, v = _qkv(hp, w, toks, pos)
-    ref = _update(hp, w, q[32:], pos[32:], k, v, pos)
+    ref = _update(hp, w, q[n:], pos[n:], k, v, pos)
     store, model = build(lstk, dev, hp, w, n_batch=T, kv_size=512)
-    run(model, 0, toks[:32], hp, dev)
+    run(model, 0, toks[:n], hp, dev)
     model.prepare(0, toks[:5])
-    _compare(_device_update(model, hp, w, 0, toks[32:], dev), ref, "hole")
+    _compare(_device_update(model, hp, w, 0, toks[n:], dev), ref, "hole")
     model.close()
     store.close()
 
@@ -166,17 +166,17 @@ def test_block_whose_first_cells_were_never_written(lstk, dev):
 def test_range_past_the_block_map(lstk, dev):
     """A sequence whose first block lies 131072 cells below the others: 2052 passes, more than the map of live blocks holds, so
     every cell of the range is visited in order, in a cache too large for the order by position."""
-    heads, hd, T, other, kv_size = (128, 32), 64, 113, 131072, 132096
+    heads, hd, T, other, kv_size, n = (128, 32), 64, 113, 131072, 132096, 96
     hp, w = _one_layer(*heads, hd)
-    cells = (32 + other + T + 255) // 256 * 256
+    cells = (n + other + T + 255) // 256 * 256
     assert lstk.attn_plan(T, *heads, hd, kv_size, cells)[2:4] == (cells, 1) and cells > 64 * 2048
-    assert lstk.attn_split(T, *heads, hd, kv_size, cells)
-    toks, pos = prompt(8, 32 + T, hp["n_vocab"]), np.arange(32 + T)
+    assert lstk.attn_split(T, *heads, hd, kv_size, cells, 0, n + T)
+    toks, pos = prompt(8, n + T, hp["n_vocab"]), np.arange(n + T)
     q, k, v = _qkv(hp, w, toks, pos)
-    ref = _update(hp, w, q[32:], pos[32:], k, v, pos)
+    ref = _update(hp, w, q[n:], pos[n:], k, v, pos)
     store, model = build(lstk, dev, hp, w, n_batch=T, kv_size=kv_size)
-    run(model, 0, toks[:32], hp, dev)
+    run(model, 0, toks[:n], hp, dev)
     model.fill_context(5, other, seed=5)
-    _compare(_device_update(model, hp, w, 0, toks[32:], dev), ref, "past the map")
+    _compare(_device_update(model, hp, w, 0, toks[n:], dev), ref, "past the map")
     model.close()
     store.close()
