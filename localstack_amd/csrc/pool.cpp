@@ -861,10 +861,11 @@ int check_call(lstk_pool *P, int layer, int T) {
 //     Q4_K gate and up, another k-quant down: 8 56 / 56 and 46 / 43, 12 69 / 66 and 57 / 44, 17 80 / 75 and 71 / 45
 //     KQ8 gate and up (Q2_K + Q3_K): 12 92 / 88 and 76 / 54, 17 107 / 102 and 92 / 56, 24 123 / 112 and 117 / 63
 //     Q8_0: 16 86 / 90 and 69 / 52, 24 102 / 101 and 90 / 60, 32 118 / 113 and 110 / 64, 48 150 / 126 and 152 / 77
-//   pairs, which pay for the launches: 64, or 96 for Q4_K experts below two million weights (fewer experts or fewer used
-//     each, even routing). 16 experts, 2 used: Q4_K 18 pairs 27 / 34, 48 35 / 35, 64 37 / 35; Q4_K + Q6_K 24 32 / 36, 64 39 / 37;
+//   pairs, which pay for the launches: 64, or 112 for experts of one to four million weights with Q4_K gate and up (160 with
+//     Q8_0 down), which the GEMV path reads fast (even routing). 16 experts, 2 used: Q4_K 18 pairs 27 / 34, 48 35 / 35, 64 37 / 35; Q4_K + Q6_K 24 32 / 36, 64 39 / 37;
 //     Q2_K + Q3_K 34 39 / 40; Q8_0 48 38 / 38, 64 40 / 39. 8 experts, 1 used: Q4_K 32 31 / 34, 48 35 / 35. 32 experts of h 1024,
-//     f 512, 4 used: Q4_K 36 27 / 31, 68 31 / 32, 96 32 / 32
+//     f 512, 4 used: Q4_K 36 27 / 31, 68 31 / 32, 96 32 / 32; of h 512, f 2048: Q4_K 64 35 / 39, 96 38 / 39, Q4_K + Q6_K 64 39 / 43,
+//     Q4_K + Q8_0 128 40 / 42; 60 experts of h 1024, f 768, 6 used: Q4_K 72 34 / 38, Q4_K + Q6_K 72 38 / 40
 //   pairs per expert (most experts then have a few): 1/2 with Q4_K experts, 3/4 with other k-quants among them, 3/2 with
 //     Q8_0 among them. 128 experts of h 1024, f 768, 1 used: Q4_K 0.38 32 / 37, Q4_K + Q6_K 0.5 40 / 41, Q2_K + Q3_K 0.5 47 / 48, Q8_0 0.5
 //     42 / 45, 0.75 58 / 60; 256 experts, 8 used: Q4_K 0.28 43 / 45, 0.38 51 / 52
@@ -877,7 +878,8 @@ bool grouped_pays(int tg, int td, long h, long f, int T, int k, int E) {
     int from = 17;
     if (weights < 1000000 || tg == lstk::kTypeQ8_0) from = 32;
     else if (tg == lstk::kTypeQ4_K) from = q4 ? 9 : td == lstk::kTypeQ8_0 ? 32 : 12;
-    if (T < from || np < (q4 && weights >= 1000000 && weights < 2000000 ? 96 : 64)) return false;
+    const bool small_q4 = tg == lstk::kTypeQ4_K && weights >= 1000000 && weights < 4000000;
+    if (T < from || np < (!small_q4 ? 64 : q8 ? 160 : 112)) return false;
     return 4 * np >= (q4 ? 2 : q8 ? 6 : 3) * (long) E;
 }
 // LSTK_GROUPED_MIN_TOKENS, or -1 where it is not set.

@@ -144,15 +144,15 @@ def test_noalloc_groups_only_in_its_own_scratch(lstk, types, h, f, E, k):
         lstk.moe_plan(types, h, f, E, k, 0)
 
 
-Q8, Q4, Q4KM, Q2XL = (8, 8, 8), (12, 12, 12), (12, 12, 14), (10, 10, 11)
+Q8, Q4, Q4KM, Q2XL, Q48 = (8, 8, 8), (12, 12, 12), (12, 12, 14), (10, 10, 11), (12, 12, 8)
 
 
 @pytest.mark.parametrize("h,f,E,k,first", [
     (2048, 768, 128, 8, {Q8: 32, Q4: 9, Q4KM: 12, Q2XL: 17}),    # the shape the token counts were measured at
     (2048, 768, 16, 2, {Q8: 32, Q4: 32, Q4KM: 32, Q2XL: 32}),    # 64 pairs (18 of Q4_K measured 27 us on the GEMV path, 34 grouped)
     (2048, 768, 8, 1, {Q8: 64, Q4: 64, Q4KM: 64, Q2XL: 64}),
-    (1024, 512, 32, 4, {Q8: 32, Q4: 24, Q4KM: 16, Q2XL: 17}),    # 96 pairs for small Q4_K experts
-    (1024, 768, 128, 1, {Q8: 192, Q4: 64, Q4KM: 96, Q2XL: 96}),  # pairs per expert
+    (1024, 512, 32, 4, {Q8: 32, Q4: 28, Q4KM: 28, Q2XL: 17, Q48: 40}),  # 112 pairs for small experts with Q4_K gate, 160 with Q8_0 down
+    (1024, 768, 128, 1, {Q8: 192, Q4: 64, Q4KM: 112, Q2XL: 96}),        # pairs per expert
     (256, 512, 8, 2, {Q8: 32, Q4: 32, Q4KM: 32, Q2XL: 32}),
 ])
 def test_grouped_path_starts_where_it_measured_no_slower(lstk, monkeypatch, h, f, E, k, first):
